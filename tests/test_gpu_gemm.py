@@ -910,3 +910,28 @@ def test_device_packer(gpu, m, n):
     want_words = oracle.pack(v)
     assert np.array_equal(dst.cpu().numpy(), want_words)
     assert np.array_equal(back.cpu().numpy(), oracle.unpack(want_words, n))
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("m, n", [(1, 1), (700, 1), (300, 3), (7, 4), (9, 5), (33, 7), (64, 32), (3, 1023), (2, 1025),
+                                  (257, 2040), (129, 261)])
+def test_device_packer_at_row_and_workgroup_ends(gpu, m, n, offset):
+    """Groups of four elements and words that cross rows, workgroups that begin and end inside a
+    row, and arrays that start on a dword but not on 16 bytes; guard words around the results."""
+    import torch
+
+    import int4linear_amd as lib
+
+    v = np.random.default_rng(31 * m + n).integers(-8, 8, size=(m, n), dtype=np.int32)
+    words = (n + 7) // 8
+    src = torch.zeros(m * n + offset, dtype=torch.int32, device="cuda:0")
+    src[offset:] = torch.from_numpy(v.reshape(-1)).to("cuda:0")
+    dst = torch.full((m * words + offset + 1,), -77, dtype=torch.int32, device="cuda:0")
+    back = torch.full((m * n + offset + 1,), -77, dtype=torch.int32, device="cuda:0")
+    lib.pack_device(src[offset:], dst[offset:], m, n)
+    lib.unpack_device(dst[offset:], back[offset:], m, n)
+    torch.cuda.synchronize()
+    for got, want in ((dst, oracle.pack(v)), (back, v)):
+        got = got.cpu().numpy()
+        assert np.array_equal(got[offset:-1], want.reshape(-1))
+        assert got[-1] == -77 and (offset == 0 or got[0] == -77)
