@@ -271,13 +271,13 @@ int run_mfma_auto(PerDevice *pd, const void *a, const void *b, void *c, int m, i
         (source == Workspace::Static && need > kStaticScratchBytes)) {
         e = launch_mfma(a, b, c, m, n, k, ep, pd->info, stream);
     } else if (source == Workspace::Static) {
-        e = launch_mfma_splitk(a, b, c, m, n, k, pd->scratch, ep, pd->info, stream);
+        e = launch_mfma_splitk(a, b, c, m, n, k, pd->scratch, pd->arrivals + kSkinnyArrivalWords, ep, pd->info, stream);
     } else {
         std::lock_guard<std::mutex> lock(pd->ws_mutex);
         void *ws = nullptr;
         if (acquire_workspace(pd, need, stream, &ws) != INT4LINEAR_OK)
             ws = nullptr;  // no workspace: the unsplit kernel
-        e = launch_mfma_splitk(a, b, c, m, n, k, ws, ep, pd->info, stream);
+        e = launch_mfma_splitk(a, b, c, m, n, k, ws, pd->arrivals, ep, pd->info, stream);
     }
     return e == hipSuccess ? INT4LINEAR_OK : fail_hip(e);
 }

@@ -144,13 +144,25 @@ hipError_t mfma_init(const DeviceInfo &dev);
 hipError_t launch_mfma(const void *a, const void *b, void *c, int m, int n, int k,
                        const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
 
-// Split-K form for shapes with few tiles and long K: ksplit K-slices per 128 x 128 tile write
-// partial sums into `workspace` (mfma_workspace_bytes() bytes, 0 = the shape is not split),
-// a second kernel adds them up and applies the epilogue.  With a null workspace it is
-// launch_mfma.
+// Split-K form for shapes with few tiles and long K, on mfma_workspace_bytes() bytes at
+// `workspace` (0 = the shape is not split): the small-grid form's split where that applies,
+// otherwise ksplit K-slices per 128 x 128 tile write partial sums and a second kernel adds them up
+// and applies the epilogue.  With a null workspace it is launch_mfma.
 size_t mfma_workspace_bytes(int m, int n, int k, const DeviceInfo &dev);
-hipError_t launch_mfma_splitk(const void *a, const void *b, void *c, int m, int n, int k, void *workspace,
+hipError_t launch_mfma_splitk(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
                               const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
+
+// Its small-grid form (kernels_grid.hip), for shapes with at most half as many 128 x 128 tiles as
+// CUs (grid_preferred).  With few tiles and long K it is split over K across workgroups:
+// grid_split_bytes() bytes of partial sums in `workspace` (8-byte aligned; 0 = the shape is not
+// split), arrivals counted at `arrivals` as by launch_skinny_ksplit below.
+hipError_t grid_init(const DeviceInfo &dev);
+bool grid_preferred(int m, int n, const DeviceInfo &dev);
+hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
+                       hipStream_t stream);
+size_t grid_split_bytes(int m, int n, int k, const DeviceInfo &dev);
+hipError_t launch_grid_split(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
+                             const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
 
 // The same kernel with the workgroup tile forced to 128 x 128 or 256 x 256 (`tile`).
 hipError_t launch_mfma_tile(const void *a, const void *b, void *c, int m, int n, int k, int tile,

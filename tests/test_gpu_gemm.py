@@ -465,6 +465,47 @@ def test_small_grid_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k, kernel="mfma")
 
 
+@pytest.mark.parametrize("m, n, k, split", [
+    # 32 x 32 tiles: stages of four pieces of 128, the last one with one, two, three or all of them
+    (70, 33, 128, False), (96, 96, 256, False), (65, 300, 896, False), (129, 511, 2048, False),
+    # 64 x 32 tiles, four waves and (K > 2048) eight
+    (257, 1000, 384, False), (640, 600, 1920, False), (257, 1000, 2176, False), (639, 601, 2432, False),
+    # 64 x 64 tiles
+    (515, 2050, 128, False), (1025, 1000, 640, False), (1000, 1111, 1152, False),
+    # each of them split over K across workgroups, with odd numbers of pieces per slice
+    (65, 200, 8448, True), (200, 700, 8960, True), (250, 2300, 12544, True), (66, 60, 8320, True)])
+def test_tiles_of_the_small_grid_form(gpu, host_threads, m, n, k, split):
+    """Every tile of the small-grid form at its edges: rows and columns past the tile, K that
+    ends inside a stage, fewer stages than the ring holds, all output types; the split over K
+    called several times (its counters go back to zero) and without a workspace."""
+    import torch
+
+    import int4linear_amd as lib
+
+    x = helpers.uniform_s4(2600 + m, m, k)
+    w = helpers.uniform_s4(2700 + n, n, k)
+    want = oracle.linear_ref(x, w, threads=host_threads)
+    xp, wp = helpers.pack_bytes(x), helpers.pack_bytes(w)
+    assert lib.kernel_for_shape(m, n, k) == "mfma"
+    assert (lib.workspace_bytes(m, n, k) > 0) == split
+    for rep in range(3 if split else 1):
+        assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="auto"), want), rep
+    rng = np.random.default_rng(m + k)
+    bias = rng.integers(-1000, 1000, size=n, dtype=np.int32)
+    rs = rng.uniform(0.1, 2.0, size=m).astype(np.float32)
+    cs = rng.uniform(0.1, 2.0, size=n).astype(np.float32)
+    xd, wd = helpers.to_device_bytes(xp), helpers.to_device_bytes(wp)
+    bd, rd, cd = (torch.from_numpy(a).to("cuda:0") for a in (bias, rs, cs))
+    y = torch.full((m, n), -1, dtype=torch.int32, device="cuda:0")
+    lib.linear_s32(xd, wd, bd, y, m, n, k)
+    assert np.array_equal(y.cpu().numpy(), oracle.epilogue(want, bias))
+    yf = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+    lib.linear_f32(xd, wd, None, rd, cd, yf, m, n, k)
+    assert np.array_equal(yf.cpu().numpy().view(np.int32), oracle.epilogue(want, None, rs, cs, f32=True).view(np.int32))
+    helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k)
+    assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="mfma"), want)  # never split
+
+
 @pytest.mark.parametrize("m, n, k", [(300, 2049, 8192), (257, 1000, 4096), (512, 1024, 14336), (300, 520, 16392),
                                      (1024, 4096, 14336)])
 def test_split_k_form_of_the_fp6_kernel(gpu, host_threads, m, n, k):
