@@ -21,7 +21,7 @@ constexpr int kMaxDevices = 64;
 // uses PerDevice::scratch.
 constexpr size_t kStaticScratchBytes = (size_t)INT4LINEAR_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
-// Arrival counters of the weight-streaming kernel's split over K (kernels.h): two sets, the
+// Arrival counters of the splits over K that meet inside a launch (kernels.h): two sets, the
 // first for calls that keep their partial sums in the internal workspace, the second for
 // int4linear_gemm_s4s4s32_static.  Zero when the library is loaded; every launch leaves them
 // zero again.
@@ -246,7 +246,7 @@ int run_fp6(PerDevice *pd, const void *a, const void *b, void *c, int m, int n, 
     if (source == Workspace::Static) {
         if (need > kStaticScratchBytes)
             return INT4LINEAR_ERR_SCRATCH;
-        e = launch_fp6(a, b, c, m, n, k, pd->scratch, ep, pd->info, stream);
+        e = launch_fp6(a, b, c, m, n, k, pd->scratch, pd->arrivals + kSkinnyArrivalWords, ep, pd->info, stream);
     } else {
         if (source == Workspace::None || capturing)
             return INT4LINEAR_ERR_UNSUPPORTED;
@@ -255,7 +255,7 @@ int run_fp6(PerDevice *pd, const void *a, const void *b, void *c, int m, int n, 
         const int st = acquire_workspace(pd, need, stream, &ws);
         if (st != INT4LINEAR_OK)
             return st;
-        e = launch_fp6(a, b, c, m, n, k, ws, ep, pd->info, stream);
+        e = launch_fp6(a, b, c, m, n, k, ws, pd->arrivals, ep, pd->info, stream);
     }
     return e == hipSuccess ? INT4LINEAR_OK : fail_hip(e);
 }

@@ -170,11 +170,10 @@ hipError_t launch_mfma_tile(const void *a, const void *b, void *c, int m, int n,
 
 // FP6-MFMA path: converts both operands into a workspace of fp6_workspace_bytes() bytes
 // (256-byte aligned), then runs the GEMM on it.  Requires K % 8 == 0, K < 2^18.  With few
-// output tiles and long K the GEMM is split over K (fp6_ksplit() slices per tile, 1 = not
-// split; it depends on the device's CU count and is 1 while that is unknown): the partial
-// sums go into slabs in the same workspace and a second kernel adds them up.
+// output tiles and long K the GEMM is split over K (it depends on the device's CU count and is
+// not while that is unknown): partial sums in the same workspace, arrivals counted at
+// `arrivals` as by launch_skinny_ksplit below.
 bool fp6_supports(int m, int n, int k);
-int fp6_ksplit(int m, int n, int k, const DeviceInfo &dev);
 size_t fp6_workspace_bytes(int m, int n, int k, const DeviceInfo &dev);
 hipError_t fp6_init(const DeviceInfo &dev);
 // The two halves of launch_fp6 on caller-owned buffers: an operand of `rows` rows converts
@@ -183,8 +182,15 @@ size_t fp6_operand_bytes(int rows, int k);
 hipError_t launch_fp6_convert(const void *src, void *dst, int rows, int k, hipStream_t stream);
 hipError_t launch_fp6_gemm(const void *a_conv, const void *b_conv, void *c, int m, int n, int k,
                            const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
-hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace,
+hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
                       const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
+// Its GEMM for grids of few tiles (kernels_fp6_grid.hip): fp6_grid_slices() slices of K across
+// workgroups with `bytes` bytes of partial sums (1 and 0: not split).
+hipError_t fp6_grid_init(const DeviceInfo &dev);
+bool fp6_grid_preferred(int m, int n, const DeviceInfo &dev);
+int fp6_grid_slices(int m, int n, int k, const DeviceInfo &dev, size_t *bytes);
+hipError_t launch_fp6_grid(const void *a_conv, const void *b_conv, void *c, int m, int n, int k, int slices, void *partial,
+                           unsigned *arrivals, const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
 
 // Weight-streaming kernel for skinny M.  K % 128 == 0; M <= 64, or more (in runs of 64
 // rows) when K splits into 128-byte tiles that fit the kernel's plans.  skinny_preferred:

@@ -24,13 +24,12 @@
 //     the workspace is already in the order lanes consume it, global->LDS is a linear
 //     direct-to-LDS copy, LDS->VGPR is one 16-byte and one 8-byte read per lane per
 //     fragment at consecutive addresses (no swizzle, no bank conflicts), and the main loop
-//     contains no VALU work at all.  With few output tiles and long K its work items are
-//     K-slices of tiles, which store partial sums into slabs of the workspace.
-//     (launch_splitk_reduce adds those slabs up and applies the epilogue).
+//     contains no VALU work at all.  (Grids of few tiles run on kernels_fp6_grid.hip.)
 //
 // Order of k inside a fragment is whatever the converter produces; it only has to be the
 // same for both operands, which it is because both go through the same converter.
 #include "kernels.h"
+#include "fp6_format.h"
 
 #include <type_traits>
 #include <utility>
@@ -50,22 +49,12 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 #define I4L_WAIT_VM(n) ((0x0F70) | ((n) & 0xF) | ((((n) >> 4) & 0x3) << 14))
 #define I4L_WAIT_LGKM0 0xC07F
 
-constexpr int kTileRows = 256;                        // rows of either operand per tile
-constexpr int kFragRows = 32;                         // rows of one MFMA operand
-constexpr int kFragK = 64;                            // k of one MFMA
-constexpr int kFragBytes = 64 * 24;                   // 64 lanes x 192 bits
-constexpr int kFragLoBytes = 64 * 16;                 // the 16-byte parts come first
-constexpr int kStageK = 128;                          // k per pipeline stage
-constexpr int kFragsK = kStageK / kFragK;             // 2
-constexpr int kFragsRows = kTileRows / kFragRows;     // 8
-constexpr int kOperandStageBytes = kFragsK * kFragsRows * kFragBytes;  // 24 KiB
 constexpr int kStageBytes = 2 * kOperandStageBytes;                    // 48 KiB
 constexpr int kStages = 3;
 constexpr int kLdsBytes = kStages * kStageBytes;                       // 144 KiB
 constexpr int kStaggerGroups = 8;                     // start groups within an XCD (power of two)
 constexpr int kStaggerTicks = 120;                    // delay between groups, in 10-ns ticks of the constant clock
 constexpr int kStaggerMinRounds = 2;                  // tiles per workgroup from which the start is staggered
-constexpr float kUnscale = 64.f;                      // the codes are n/8: a product is n*m/64
 
 // ---- converter --------------------------------------------------------------------------
 
@@ -109,6 +98,8 @@ struct ConvertJob {
     int row_blocks;       // 32-row blocks including the padding
 };
 
+typedef v4i v4i_dword_aligned __attribute__((aligned(4)));
+
 constexpr int kConvK = 512;                          // k per converter workgroup
 constexpr int kConvFrags = kConvK / kFragK;          // 8 fragments out
 constexpr int kConvChunks = kConvK / 32;             // 16-byte input chunks per row
@@ -148,11 +139,15 @@ __global__ __launch_bounds__(256) void fp6_convert_kernel(ConvertJob ja, Convert
         if (ALIGNED16) {
             if (row < job.rows && k0 < k)
                 w[h] = __builtin_nontemporal_load((const v4i *)src);
-        } else {
+        } else if (row < job.rows) {
+            if (k0 + 32 <= k) {
+                w[h] = *(const v4i_dword_aligned *)src;
+            } else {
 #pragma unroll
-            for (int d = 0; d < 4; ++d)
-                if (row < job.rows && k0 + 8 * d < k)
-                    w[h][d] = *(const int *)(src + 4 * d);
+                for (int d = 0; d < 3; ++d)
+                    if (k0 + 8 * d < k)
+                        w[h][d] = *(const int *)(src + 4 * d);
+            }
         }
     }
 #pragma unroll
@@ -263,7 +258,7 @@ struct WholeKernel {
 template <class C, bool HALF_OUT = false, class Parts = WholeKernel>
 __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
     const uint8_t *__restrict__ XW, const uint8_t *__restrict__ WW, int32_t *__restrict__ Y,
-    int M, int N, int K, int tiles_m, int tiles_n, int ksplit, Epilogue ep)
+    int M, int N, int K, int tiles_m, int tiles_n, Epilogue ep)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
@@ -271,17 +266,11 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::WAVES_N;
     const int wn = wave % C::WAVES_N;
-    // With ksplit > 1 a work item is one K-slice of one tile: item v is slice v / tiles of
-    // tile v % tiles (so the items of one slice are laid out like the tiles of an unsplit
-    // launch), covers KT of the KT_all stages, and stores its plain partial sums into slab
-    // `slice` of Y (M * N int32 each), which a second kernel adds up.
-    const int KT_all = K / kStageK;
-    const int KT = KT_all / ksplit;
-    const int tiles = tiles_m * tiles_n;
-    const int total_tiles = tiles * ksplit;  // work items
+    const int KT = K / kStageK;
+    const int total_tiles = tiles_m * tiles_n;
     const int nblk = gridDim.x;
     const int bid = blockIdx.x;
-    const bool ep_plain = !HALF_OUT && (ksplit > 1 || (!ep.bias && !ep.row_scale && !ep.col_scale && !ep.out));
+    const bool ep_plain = !HALF_OUT && !ep.bias && !ep.row_scale && !ep.col_scale && !ep.out;
     if (bid >= total_tiles)
         return;
     const int my_tiles = (total_tiles - bid + nblk - 1) / nblk;
@@ -301,13 +290,11 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
 
     auto ld_setup_tile = [&](int it) {
         int tm, tn;
-        const int item = bid + it * nblk;
-        const int slice = item / tiles;
-        tile_coords(item - slice * tiles, tiles, tiles_m, tiles_n, tm, tn);
+        tile_coords(bid + it * nblk, total_tiles, tiles_m, tiles_n, tm, tn);
         if constexpr (!Parts::kOwnTile)
             tm = tn = 0;
-        xptr = XW + ((size_t)tm * KT_all + (size_t)slice * KT) * kOperandStageBytes;
-        wptr = WW + ((size_t)tn * KT_all + (size_t)slice * KT) * kOperandStageBytes;
+        xptr = XW + (size_t)tm * KT * kOperandStageBytes;
+        wptr = WW + (size_t)tn * KT * kOperandStageBytes;
     };
     auto ld_chunk = [&](auto c, unsigned ring) {  // c < CH/2: X half, else W half; ring: the buffer's offset
         constexpr int cc = decltype(c)::value;
@@ -517,13 +504,11 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
             //   m = 32*j + 8*(t/4) + 4*(lane/32) + t%4,  n = 32*i + lane%32,
             // so one dword store writes two rows of 32 consecutive n (128 B each).
             int tm, tn;
-            const int item = bid + cur_it * nblk;
-            const int slice = item / tiles;
-            tile_coords(item - slice * tiles, tiles, tiles_m, tiles_n, tm, tn);
+            tile_coords(bid + cur_it * nblk, total_tiles, tiles_m, tiles_n, tm, tn);
             const int m0 = tm * kTileRows, n0 = tn * kTileRows;
             const int rows_left = M - m0;  // > 0
             const int cols_left = N - n0;  // > 0
-            int32_t *ybase = Y + (size_t)slice * (size_t)M * (size_t)N + (size_t)m0 * N + n0;
+            int32_t *ybase = Y + (size_t)m0 * N + n0;
             const size_t slab_rows = rows_left < kTileRows ? rows_left : kTileRows;
             const size_t extent = ((slab_rows - 1) * (size_t)N + (size_t)(cols_left < kTileRows ? cols_left : kTileRows)) * 4u;
             __amdgpu_buffer_rsrc_t rsrc =
@@ -591,8 +576,7 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
                     }
                 } else {
                     // The half-width kinds: a descriptor over the same tile of an output of
-                    // two-byte elements, every offset halved (no K-slices here: an epilogue
-                    // goes with ksplit == 1, Y is the output's base).
+                    // two-byte elements, every offset halved.
                     __amdgpu_buffer_rsrc_t rsrc16 = __builtin_amdgcn_make_buffer_rsrc(
                         (uint8_t *)Y + ((size_t)m0 * N + n0) * 2u, 0, (int)(extent / 2u), 0x00020000);
 #pragma unroll
@@ -659,32 +643,24 @@ bool fp6_supports(int m, int n, int k)
     return m >= 1 && n >= 1 && m <= kMaxRows && n <= kMaxRows && k >= 8 && k % 8 == 0 && k <= (1 << 18) - kStageK;
 }
 
-int fp6_ksplit(int m, int n, int k, const DeviceInfo &dev)
-{
-    const long tiles = (long)((m + kTileRows - 1) / kTileRows) * ((n + kTileRows - 1) / kTileRows);
-    const int stages = (k + kStageK - 1) / kStageK;
-    // Measured: two slices of 128 tiles gain nothing over 128 unsplit tiles (the second kernel
-    // and the slabs cost what the idle half of the device did); four of 64 tiles gain 9-16 %.
-    if (dev.cu_count <= 0 || tiles * 4 > dev.cu_count)
-        return 1;
-    // The most slices that still leave a workgroup per CU, 2048 k per slice and equal slices.
-    for (int ks : {8, 7, 6, 5, 4, 3, 2})
-        if (tiles * ks <= dev.cu_count && stages % ks == 0 && stages / ks >= 16)
-            return ks;
-    return 1;
-}
-
 size_t fp6_workspace_bytes(int m, int n, int k, const DeviceInfo &dev)
 {
-    const int ks = fp6_ksplit(m, n, k, dev);
-    return operand_ws_bytes(m, k) + operand_ws_bytes(n, k) + (ks > 1 ? (size_t)ks * (size_t)m * (size_t)n * 4u : 0);
+    // (partial sums: whole multiples of the output's size)
+    const size_t out = (size_t)m * (size_t)n * 4u;
+    size_t partial = 0;
+    if (dev.cu_count > 0)
+        fp6_grid_slices(m, n, k, dev, &partial);
+    return operand_ws_bytes(m, k) + operand_ws_bytes(n, k) + (partial + out - 1) / out * out;
 }
 
 hipError_t fp6_init(const DeviceInfo &dev)
 {
     if (dev.lds_per_cu < kLdsBytes)
         return hipErrorInvalidConfiguration;
-    hipError_t e = hipFuncSetAttribute((const void *)fp6_gemm_kernel<Fp6Cfg>,
+    hipError_t e = fp6_grid_init(dev);
+    if (e != hipSuccess)
+        return e;
+    e = hipFuncSetAttribute((const void *)fp6_gemm_kernel<Fp6Cfg>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     if (e != hipSuccess)
         return e;
@@ -696,10 +672,12 @@ size_t fp6_operand_bytes(int rows, int k) { return operand_ws_bytes(rows, k); }
 
 namespace {
 
-ConvertJob make_job(const void *src, void *dst, int rows)
+// whole_tiles: rows of zeros up to the next multiple of 256 are written as well (the large GEMM
+// kernel reads them, the small-grid one reads 64-row pairs at most).
+ConvertJob make_job(const void *src, void *dst, int rows, bool whole_tiles = true)
 {
-    const int tiles = (rows + kTileRows - 1) / kTileRows;
-    return ConvertJob{(const uint8_t *)src, (uint8_t *)dst, rows, tiles * kFragsRows};
+    const int unit = whole_tiles ? kTileRows : 2 * kFragRows;
+    return ConvertJob{(const uint8_t *)src, (uint8_t *)dst, rows, (rows + unit - 1) / unit * (unit / kFragRows)};
 }
 
 int padded_k(int k) { return (k + kStageK - 1) / kStageK * kStageK; }
@@ -729,28 +707,21 @@ hipError_t launch_fp6_convert(const void *src, void *dst, int rows, int k, hipSt
 
 namespace {
 
-// ksplit > 1: `c` is ksplit slabs of m * n partial sums and `ep` must be empty.
-hipError_t launch_gemm_items(const void *a_conv, const void *b_conv, void *c, int m, int n, int k, int ksplit,
-                             const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
+hipError_t launch_tiles(const void *a_conv, const void *b_conv, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
+                        hipStream_t stream)
 {
     using C = Fp6Cfg;
     const int tiles_m = (m + kTileRows - 1) / kTileRows;
     const int tiles_n = (n + kTileRows - 1) / kTileRows;
-    const long total = (long)tiles_m * tiles_n * ksplit;
+    const long total = (long)tiles_m * tiles_n;
     if (total > 0x7fffffffL || (size_t)kTileRows * (size_t)n * 4u > 0x40000000ull)
         return hipErrorInvalidValue;
     long grid = (long)dev.cu_count * C::OCC;
     if (grid > total)
         grid = total;
-    if (ep.out >= kOutF16) {
-        if (ksplit != 1)
-            return hipErrorInvalidValue;
-        fp6_gemm_kernel<C, true><<<(unsigned)grid, C::THREADS, kLdsBytes, stream>>>(
-            (const uint8_t *)a_conv, (const uint8_t *)b_conv, (int32_t *)c, m, n, padded_k(k), tiles_m, tiles_n, ksplit, ep);
-    } else {
-        fp6_gemm_kernel<C><<<(unsigned)grid, C::THREADS, kLdsBytes, stream>>>(
-            (const uint8_t *)a_conv, (const uint8_t *)b_conv, (int32_t *)c, m, n, padded_k(k), tiles_m, tiles_n, ksplit, ep);
-    }
+    auto *kern = ep.out >= kOutF16 ? fp6_gemm_kernel<C, true> : fp6_gemm_kernel<C>;
+    kern<<<(unsigned)grid, C::THREADS, kLdsBytes, stream>>>((const uint8_t *)a_conv, (const uint8_t *)b_conv, (int32_t *)c, m, n,
+                                                             padded_k(k), tiles_m, tiles_n, ep);
     return hipGetLastError();
 }
 
@@ -759,27 +730,26 @@ hipError_t launch_gemm_items(const void *a_conv, const void *b_conv, void *c, in
 hipError_t launch_fp6_gemm(const void *a_conv, const void *b_conv, void *c, int m, int n, int k,
                            const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
 {
-    return launch_gemm_items(a_conv, b_conv, c, m, n, k, 1, ep, dev, stream);
+    if (fp6_grid_preferred(m, n, dev))
+        return launch_fp6_grid(a_conv, b_conv, c, m, n, k, 1, nullptr, nullptr, ep, dev, stream);
+    return launch_tiles(a_conv, b_conv, c, m, n, k, ep, dev, stream);
 }
 
-hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace,
+hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
                       const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
 {
     uint8_t *xws = (uint8_t *)workspace;
     uint8_t *wws = xws + operand_ws_bytes(m, k);
-    hipError_t e = launch_convert_jobs(make_job(a, xws, m), make_job(b, wws, n), k, stream);
+    const bool grid = fp6_grid_preferred(m, n, dev);
+    hipError_t e = launch_convert_jobs(make_job(a, xws, m, !grid), make_job(b, wws, n, !grid), k, stream);
     if (e != hipSuccess)
         return e;
-    // Few tiles and long K: K-slices of every tile on their own CUs, partial sums in slabs
-    // behind the operands, a second kernel for the sum and the epilogue.
-    const int ks = fp6_ksplit(m, n, k, dev);
-    if (ks == 1)
-        return launch_gemm_items(xws, wws, c, m, n, k, 1, ep, dev, stream);
-    int32_t *slabs = (int32_t *)(wws + operand_ws_bytes(n, k));
-    e = launch_gemm_items(xws, wws, slabs, m, n, k, ks, Epilogue{}, dev, stream);
-    if (e != hipSuccess)
-        return e;
-    return launch_splitk_reduce(slabs, c, (size_t)m * (size_t)n, ks, n, ep, stream);
+    if (!grid)
+        return launch_tiles(xws, wws, c, m, n, k, ep, dev, stream);
+    // Few tiles and long K: slices of K across workgroups, partial sums behind the operands.
+    size_t partial = 0;
+    const int slices = fp6_grid_slices(m, n, k, dev, &partial);
+    return launch_fp6_grid(xws, wws, c, m, n, k, slices, wws + operand_ws_bytes(n, k), arrivals, ep, dev, stream);
 }
 
 }  // namespace int4linear

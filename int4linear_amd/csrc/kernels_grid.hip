@@ -9,7 +9,7 @@
 //     several MFMAs: 6 vector operations per MFMA instead of the 12 of 32 x 32 quadrants, where
 //     the vector unit, not the matrix unit, sets the pace.  The sums meet in LDS at the end: each
 //     wave collects one part of the tile and stores it.
-//   * a stage is 256 or 512 of K: whole 128-byte lines of every row, one barrier.
+//   * a stage is 512 of K: whole 128-byte lines of every row, one barrier.
 //   * one set of packed and of widened operands is a pipeline: the even-nibble MFMAs of a unit run
 //     while its odd nibbles are masked, its odd-nibble MFMAs while the next unit's even nibbles
 //     are shifted and masked.  No registers for a second set, so three waves fit a SIMD.
@@ -22,10 +22,7 @@
 //
 // With few tiles and long K a tile's K is split over workgroups as well; they exchange partial sums
 // through memory inside the same launch (see the kernel's end).
-#include "kernels.h"
-
-#include <type_traits>
-#include <utility>
+#include "grid_tail.h"
 
 namespace int4linear {
 
@@ -33,7 +30,6 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef unsigned long long u64;
 
 #define I4L_LDS(p) ((__attribute__((address_space(3))) void *)(p))
 // s_waitcnt immediate: vmcnt only, the other counters left at "no wait"; and lgkmcnt(0) only
@@ -57,32 +53,15 @@ __device__ __forceinline__ void wait_vm()
     __builtin_amdgcn_s_waitcnt(I4L_VMCNT(N));
 }
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F &&f)
-{
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-        (f(std::integral_constant<int, I>{}), ...);
-    }(std::make_integer_sequence<int, N>{});
-}
-
-// A wave-uniform value that the compiler may hold on the vector side, in scalar registers.
-__device__ __forceinline__ unsigned uniform(unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane((int)v); }
-__device__ __forceinline__ const uint8_t *uniform(const uint8_t *p)
-{
-    const u64 v = (u64)p;
-    return (const uint8_t *)((u64)uniform((unsigned)v) | ((u64)uniform((unsigned)(v >> 32)) << 32));
-}
-
 constexpr int kPieceK = 128;  // K comes in pieces of 128: 64 bytes of a row
-constexpr int kFrag = 32;     // rows of an MFMA 32x32x32 operand
-constexpr int kMaxSlices = 8; // of K, over workgroups
+constexpr int kFrag = kGridFrag;
 
-// KG waves share a tile of FM x FN fragments; each takes 1 / KG of every stage's K.  A stage is
-// PIECES pieces of every row, NSTAGE of them ring in LDS.
-template <int FM_, int FN_, int KG_, int PIECES_, int NSTAGE_, int WAVES_PER_SIMD_>
+// KG waves share a tile of FM x FN fragments; each takes 1 / KG of every stage's K.  NSTAGE stages
+// ring in LDS.
+template <int FM_, int FN_, int KG_, int NSTAGE_, int WAVES_PER_SIMD_>
 struct GridTile {
-    static constexpr int FM = FM_, FN = FN_, KG = KG_, PIECES = PIECES_, NSTAGE = NSTAGE_, OCC = WAVES_PER_SIMD_;
+    static constexpr int FM = FM_, FN = FN_, KG = KG_, NSTAGE = NSTAGE_, OCC = WAVES_PER_SIMD_;
+    static constexpr int PIECES = 4;                    // of every row in a stage
     static constexpr int THREADS = KG * 64;
     static constexpr int BM = FM * kFrag, BN = FN * kFrag;
     static constexpr int ROW_BYTES = 64 * PIECES;       // of a row in a stage
@@ -92,34 +71,17 @@ struct GridTile {
     static constexpr int LDS_BYTES = STAGE_BYTES * NSTAGE;
     static constexpr int CH = (BM + BN) / LOAD_ROWS / KG;  // loads per wave and stage
     static constexpr int STEPS = 2 * PIECES / KG;          // units of 64 k per wave and stage
-    static constexpr int KEEP = FM * FN * 16 / KG;         // sums per lane that a wave collects in the end
-    static_assert(PIECES == 2 || PIECES == 4, "rows of 128 or 256 bytes");
+    template <bool HALF_OUT>
+    using Tail = GridTail<FM, FN, KG, HALF_OUT>;
     static_assert((BM + BN) / LOAD_ROWS % KG == 0, "loads split evenly");
     static_assert(STEPS == 1 || STEPS == 2, "");
-    static_assert(KEEP % 2 == 0 && (KEEP <= 16 ? 16 % KEEP == 0 : KEEP % 16 == 0), "parts of fragments or whole ones");
-    static_assert(KG * (KG - 1) * KEEP * 256 <= LDS_BYTES, "the sums meet in the ring's LDS");
+    static_assert(Tail<false>::LDS_BYTES <= LDS_BYTES, "the sums meet in the ring's LDS");
     static_assert((NSTAGE - 1) * CH <= 63, "vmcnt is six bits");
     // LDS slot of 16-byte chunk c of row r is c ^ swizzle(r): sixteen lanes that read one chunk of
     // sixteen consecutive rows hit sixteen different 16-byte groups of the banks (no conflicts
     // counted).
-    __device__ static int swizzle(int r) { return PIECES == 2 ? (r >> 1) & 7 : r & 15; }
+    __device__ static int swizzle(int r) { return r & 15; }
 };
-
-// XCD-aware tile order, as in kernels_mfma.hip.
-__device__ __forceinline__ void tile_coords(int v, int total, int tiles_m, int tiles_n, int &tm, int &tn)
-{
-    constexpr int kXcd = 8, kGroup = 8;
-    const int x = v % kXcd, j = v / kXcd;
-    const int cnt = total / kXcd, rem = total % kXcd;
-    const int q = x * cnt + (x < rem ? x : rem) + j;
-    const int per_group = kGroup * tiles_n;
-    const int group = q / per_group;
-    const int first_m = group * kGroup;
-    const int gsz = (tiles_m - first_m < kGroup) ? (tiles_m - first_m) : kGroup;
-    const int in_group = q % per_group;
-    tm = first_m + in_group % gsz;
-    tn = in_group / gsz;
-}
 
 // One argument instead of eleven: the host's cost of a launch grows with their number.
 struct GridArgs {
@@ -152,7 +114,7 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void mfma_grid_kernel(GridArgs 
     const int last_pieces = pieces - (KT - 1) * C::PIECES;  // in the last stage
     const bool ragged = last_pieces != C::PIECES;
     int tm, tn;
-    tile_coords(tile, tiles, tiles_m, tiles_n, tm, tn);
+    grid_tile_coords(tile, tiles, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * C::BM, n0 = tn * C::BN;
 
     // ---- loads.  A stage is the tile's rows of X, then those of W; lane p of a load lands at byte
@@ -192,43 +154,14 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void mfma_grid_kernel(GridArgs 
     };
     issue(0, 0);
 
-    // ---- The sums this wave collects in the end are those with linear index (j * FN + i) * 16 + t
-    //      in [wave * KEEP, (wave + 1) * KEEP), accumulator t of fragment (i, j) being row
-    //      32 j + 8 (t / 4) + 4 (lane / 32) + t % 4, column 32 i + lane % 32 of the tile (X is the
-    //      MFMA A operand).  Their epilogue operands are fetched now.
-    const int fr = lane & 31;
-    const int fg = lane >> 5;
-    constexpr int kCols = C::KEEP > 16 ? C::KEEP / 16 : 1;  // fragments they come from
-    auto row_of = [&](int q) {
-        const int r = wave * C::KEEP + q, t = r % 16;
-        return r / 16 / C::FN * kFrag + 8 * (t / 4) + 4 * fg + t % 4;
-    };
-    auto col_of = [&](int i) { return (wave * C::KEEP / 16 + i) % C::FN * kFrag + fr; };
-    int bias_v[kCols];
-    float cs_v[kCols], rs_v[C::KEEP];
-#pragma unroll
-    for (int i = 0; i < kCols; ++i) {
-        bias_v[i] = 0;
-        cs_v[i] = 1.f;
-    }
-#pragma unroll
-    for (int q = 0; q < C::KEEP; ++q)
-        rs_v[q] = 1.f;
-    if (ep.bias) {
-#pragma unroll
-        for (int i = 0; i < kCols; ++i)
-            bias_v[i] = ep.bias[min(n0 + col_of(i), N - 1)];
-    }
-    if (ep.col_scale) {
-#pragma unroll
-        for (int i = 0; i < kCols; ++i)
-            cs_v[i] = ep.col_scale[min(n0 + col_of(i), N - 1)];
-    }
-    if (ep.row_scale) {
-#pragma unroll
-        for (int q = 0; q < C::KEEP; ++q)
-            rs_v[q] = ep.row_scale[min(m0 + row_of(q), M - 1)];
-    }
+    typename C::template Tail<HALF_OUT> tail;
+    tail.lane = lane;
+    tail.wave = wave;
+    tail.m0 = m0;
+    tail.n0 = n0;
+    tail.M = M;
+    tail.N = N;
+    tail.fetch(ep);
 #pragma unroll
     for (int st = 1; st < C::NSTAGE; ++st)
         if (st < KT)
@@ -237,6 +170,8 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void mfma_grid_kernel(GridArgs 
     // ---- math.  A unit is 64 k: two 16-byte chunks of a row, one per half of the wave; the even
     //      nibbles of a chunk feed one MFMA, the odd ones another.  This wave's units of a stage
     //      are wave * STEPS, ...
+    const int fr = lane & 31;
+    const int fg = lane >> 5;
     unsigned rd[C::STEPS];
 #pragma unroll
     for (int s = 0; s < C::STEPS; ++s)
@@ -355,111 +290,22 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void mfma_grid_kernel(GridArgs 
         hi_phase(std::false_type{});
     }
 
-    // ---- the sums meet in LDS: [collecting wave][sending wave][KEEP] x 64 lanes
-    __builtin_amdgcn_s_waitcnt(I4L_LGKM0);
+    __builtin_amdgcn_s_waitcnt(I4L_LGKM0);  // every wave is done with the ring
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    int kept[C::KEEP];
-    int *const area = (int *)lds + lane;
-    static_for<C::KG>([&](auto me_tag) {
-        constexpr int me = decltype(me_tag)::value;
-        if (wave == me) {
-            static_for<C::KG>([&](auto to_tag) {
-                constexpr int to = decltype(to_tag)::value;
-                static_for<C::KEEP>([&](auto q) {
-                    constexpr int r = to * C::KEEP + decltype(q)::value;
-                    const int sum = acc[r / 16 % C::FN][r / 16 / C::FN][r % 16];
-                    if constexpr (to == me)
-                        kept[q()] = sum;
-                    else
-                        area[((to * (C::KG - 1) + (me < to ? me : me - 1)) * C::KEEP + q()) * 64] = sum;
-                });
-            });
-        }
-    });
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < C::KEEP; ++q) {
-#pragma unroll
-        for (int g = 0; g < C::KG - 1; ++g)
-            kept[q] += area[((wave * (C::KG - 1) + g) * C::KEEP + q) * 64];
-        kept[q] >>= 8;  // both operands carried a factor 16 (exact for every slice of K: each product is a multiple of 256)
-    }
-
-    // ---- slices of K: every wave leaves its sums in the slab of (tile, slice), waits until they
-    //      have been acknowledged and counts itself in at the counter of (tile, wave).  The waves
-    //      with one number hold the same sums in every slice's workgroup, so the last of them to
-    //      arrive adds the others' up, stores, and puts the counter back to zero.  Nobody waits for
-    //      anybody, and integer sums do not depend on who arrives when.  (Relaxed atomic operations
-    //      at device scope go through to the level all workgroups share; fences at that scope
-    //      would write back and invalidate the XCD's whole L2 instead.)
-    if (slices > 1) {
-        constexpr int kWords = C::KEEP / 2;
-        u64 *const slabs = (u64 *)args.partial + (size_t)tile * slices * C::KG * kWords * 64 + (size_t)wave * kWords * 64 + lane;
-        constexpr int kSlab = C::KG * kWords * 64;
-#pragma unroll
-        for (int q = 0; q < kWords; ++q)
-            __hip_atomic_store(slabs + slice * kSlab + q * 64, (u64)(unsigned)kept[2 * q] | ((u64)(unsigned)kept[2 * q + 1] << 32),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        unsigned *const counter = args.arrivals + tile * C::KG + wave;
-        unsigned before = 0;
-        if (lane == 0)
-            before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        before = uniform(before);
-        if (before != (unsigned)(slices - 1))
-            return;
-        if (lane == 0)
-            __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        u64 got[kMaxSlices - 1][kWords];  // all loads go out together
-#pragma unroll
-        for (int p = 0; p < kMaxSlices - 1; ++p)
-#pragma unroll
-            for (int q = 0; q < kWords; ++q)
-                got[p][q] = p < slices - 1 ? __hip_atomic_load(slabs + (p < slice ? p : p + 1) * kSlab + q * 64, __ATOMIC_RELAXED,
-                                                               __HIP_MEMORY_SCOPE_AGENT)
-                                           : 0ull;
-#pragma unroll
-        for (int p = 0; p < kMaxSlices - 1; ++p)
-#pragma unroll
-            for (int q = 0; q < kWords; ++q) {
-                kept[2 * q] += (int)(unsigned)got[p][q];
-                kept[2 * q + 1] += (int)(unsigned)(got[p][q] >> 32);
-            }
-    }
-
-    // ---- store: 32 lanes write 32 consecutive columns.  Through a descriptor over the tile's
-    //      rows: a lane outside the matrix gets an offset beyond it and the hardware drops the
-    //      store.
-    constexpr unsigned kElem = HALF_OUT ? 2u : 4u;
-    const bool plain = !ep.bias && !ep.out;
-    const int rows_left = M - m0, cols_left = N - n0;
-    const size_t extent = ((size_t)(min(rows_left, C::BM) - 1) * N + min(cols_left, C::BN)) * kElem;
-    __amdgpu_buffer_rsrc_t rsrc =
-        __builtin_amdgcn_make_buffer_rsrc((uint8_t *)args.y + ((size_t)m0 * N + n0) * kElem, 0, (int)extent, 0x00020000);
-    unsigned col_off[kCols];
-#pragma unroll
-    for (int i = 0; i < kCols; ++i)
-        col_off[i] = col_of(i) < cols_left ? (unsigned)col_of(i) * kElem : 0x40000000u;
-#pragma unroll
-    for (int q = 0; q < C::KEEP; ++q) {
-        const unsigned off = (row_of(q) < rows_left ? (unsigned)row_of(q) * (unsigned)N * kElem : 0x80000000u) + col_off[q / 16];
-        if constexpr (HALF_OUT)
-            __builtin_amdgcn_raw_buffer_store_b16(
-                (unsigned short)epilogue_value16(ep, kept[q], bias_v[q / 16], rs_v[q], cs_v[q / 16]), rsrc, off, 0, 0);
-        else
-            __builtin_amdgcn_raw_buffer_store_b32(
-                (unsigned)(plain ? kept[q] : epilogue_value32(ep, kept[q], bias_v[q / 16], rs_v[q], cs_v[q / 16])), rsrc, off, 0, 0);
-    }
+    // (both operands carried a factor 16: every product, and with it every wave's share, is a
+    // multiple of 256)
+    tail.collect(lds, [&](auto i, auto j, auto t) { return acc[i()][j()][t()] >> 8; });
+    if (slices > 1 && !tail.exchange(args.partial, args.arrivals, tile, slice, slices))
+        return;
+    tail.store(ep, args.y);
 }
 
 // The tiles, smallest grids first.
-using Tile32x32 = GridTile<1, 1, 8, 4, 4, 2>;        // 64 KiB of LDS
-using Tile64x32Short = GridTile<2, 1, 4, 4, 3, 2>;   // 72 KiB; four waves: less to bring together at the end
-using Tile64x32Long = GridTile<2, 1, 8, 4, 3, 4>;    // 72 KiB; eight waves
-using Tile64x64 = GridTile<2, 2, 4, 4, 2, 2>;        // 64 KiB
-
-long tiles_of(int m, int n, int bm, int bn) { return (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
+using Tile32x32 = GridTile<1, 1, 8, 4, 2>;        // 64 KiB of LDS
+using Tile64x32Short = GridTile<2, 1, 4, 3, 2>;   // 72 KiB; four waves: less to bring together at the end
+using Tile64x32Long = GridTile<2, 1, 8, 3, 4>;    // 72 KiB; eight waves
+using Tile64x64 = GridTile<2, 2, 4, 2, 2>;        // 64 KiB
 
 enum class Tile { k32x32, k64x32Short, k64x32Long, k64x64 };
 
@@ -470,9 +316,9 @@ enum class Tile { k32x32, k64x32Short, k64x32Long, k64x64 };
 // 2048 4.83 / 4.82 with four / eight; 200 x 2000 x 512 3.5 / 3.9; 65 x 4096 x 4096 7.1 / 6.5).
 Tile choose_tile(int m, int n, int k, const DeviceInfo &dev)
 {
-    if (tiles_of(m, n, 32, 32) <= dev.cu_count)
+    if (grid_tiles(m, n, 32, 32) <= dev.cu_count)
         return Tile::k32x32;
-    if (tiles_of(m, n, 64, 32) <= dev.cu_count)
+    if (grid_tiles(m, n, 64, 32) <= dev.cu_count)
         return k > 2048 ? Tile::k64x32Long : Tile::k64x32Short;
     return Tile::k64x64;
 }
@@ -496,18 +342,18 @@ SplitPlan plan_split(int m, int n, int k, const DeviceInfo &dev)
     if (pieces < kMinPieces)
         return p;
     long tiles, most, waves, area;
-    if (tiles_of(m, n, 32, 32) * 4 <= dev.cu_count) {
+    if (grid_tiles(m, n, 32, 32) * 4 <= dev.cu_count) {
         p.tile = Tile::k32x32;
-        tiles = tiles_of(m, n, 32, 32), most = dev.cu_count, waves = Tile32x32::KG, area = 32 * 32;
-    } else if (tiles_of(m, n, 64, 32) * 2 <= dev.cu_count) {
+        tiles = grid_tiles(m, n, 32, 32), most = dev.cu_count, waves = Tile32x32::KG, area = 32 * 32;
+    } else if (grid_tiles(m, n, 64, 32) * 2 <= dev.cu_count) {
         p.tile = Tile::k64x32Long;
-        tiles = tiles_of(m, n, 64, 32), most = dev.cu_count, waves = Tile64x32Long::KG, area = 64 * 32;
+        tiles = grid_tiles(m, n, 64, 32), most = dev.cu_count, waves = Tile64x32Long::KG, area = 64 * 32;
     } else {
-        tiles = tiles_of(m, n, 64, 64), most = 2l * dev.cu_count, waves = Tile64x64::KG, area = 64 * 64;
+        tiles = grid_tiles(m, n, 64, 64), most = 2l * dev.cu_count, waves = Tile64x64::KG, area = 64 * 64;
     }
     if (tiles * waves > kSkinnyArrivalWords)
         return p;
-    for (int d = 2; d <= kMaxSlices && tiles * d <= most; ++d)
+    for (int d = 2; d <= kGridMaxSlices && tiles * d <= most; ++d)
         if (pieces % d == 0 && pieces / d >= kMinPiecesPerSlice)
             p.slices = d;
     if (p.slices > 1)
@@ -524,21 +370,12 @@ hipError_t init_tile()
     return e;
 }
 
-struct Split {
-    int slices = 1;
-    void *partial = nullptr;
-    unsigned *arrivals = nullptr;
-};
-
 template <class C>
-hipError_t launch_tile(const void *a, const void *b, void *c, int m, int n, int k, const Split &split, const Epilogue &ep,
+hipError_t launch_tile(const void *a, const void *b, void *c, int m, int n, int k, const GridSplit &split, const Epilogue &ep,
                        hipStream_t stream)
 {
     const int tiles_m = (m + C::BM - 1) / C::BM, tiles_n = (n + C::BN - 1) / C::BN;
-    // what the kernel assumes of a split: slices of whole pieces, a counter for every (tile, wave)
-    if (split.slices > 1 &&
-        (split.slices > kMaxSlices || k / kPieceK % split.slices != 0 || !split.partial || !split.arrivals ||
-         (long)tiles_m * tiles_n * C::KG > kSkinnyArrivalWords))
+    if (!grid_split_valid(split, (long)tiles_m * tiles_n, C::KG, k / kPieceK))
         return hipErrorInvalidValue;
     auto *kern = ep.out >= kOutF16 ? mfma_grid_kernel<C, true> : mfma_grid_kernel<C, false>;
     kern<<<(unsigned)(tiles_m * tiles_n * split.slices), C::THREADS, C::LDS_BYTES, stream>>>(
@@ -546,7 +383,7 @@ hipError_t launch_tile(const void *a, const void *b, void *c, int m, int n, int 
     return hipGetLastError();
 }
 
-hipError_t launch(Tile tile, const void *a, const void *b, void *c, int m, int n, int k, const Split &split, const Epilogue &ep,
+hipError_t launch(Tile tile, const void *a, const void *b, void *c, int m, int n, int k, const GridSplit &split, const Epilogue &ep,
                   hipStream_t stream)
 {
     switch (tile) {
@@ -575,12 +412,12 @@ hipError_t grid_init(const DeviceInfo &)
     return e;
 }
 
-bool grid_preferred(int m, int n, const DeviceInfo &dev) { return tiles_of(m, n, 128, 128) * 2 <= dev.cu_count; }
+bool grid_preferred(int m, int n, const DeviceInfo &dev) { return grid_tiles(m, n, 128, 128) * 2 <= dev.cu_count; }
 
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
                        hipStream_t stream)
 {
-    return launch(choose_tile(m, n, k, dev), a, b, c, m, n, k, Split{}, ep, stream);
+    return launch(choose_tile(m, n, k, dev), a, b, c, m, n, k, GridSplit{}, ep, stream);
 }
 
 size_t grid_split_bytes(int m, int n, int k, const DeviceInfo &dev)
@@ -592,7 +429,7 @@ hipError_t launch_grid_split(const void *a, const void *b, void *c, int m, int n
                              const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
 {
     const SplitPlan p = plan_split(m, n, k, dev);
-    return launch(p.tile, a, b, c, m, n, k, Split{p.slices, workspace, arrivals}, ep, stream);
+    return launch(p.tile, a, b, c, m, n, k, GridSplit{p.slices, workspace, arrivals}, ep, stream);
 }
 
 }  // namespace int4linear

@@ -80,11 +80,11 @@ double time_build(const uint8_t *xw, const uint8_t *ww, int32_t *y, int m, int n
     CHECK(hipEventCreate(&e0));
     CHECK(hipEventCreate(&e1));
     for (int i = 0; i < warmup; ++i)
-        kern<<<(unsigned)grid, C::THREADS, kLdsBytes, 0>>>(xw, ww, y, m, n, padded_k(k), tiles_m, tiles_n, 1, Epilogue{});
+        kern<<<(unsigned)grid, C::THREADS, kLdsBytes, 0>>>(xw, ww, y, m, n, padded_k(k), tiles_m, tiles_n, Epilogue{});
     CHECK(hipDeviceSynchronize());
     CHECK(hipEventRecord(e0, 0));
     for (int i = 0; i < iters; ++i)
-        kern<<<(unsigned)grid, C::THREADS, kLdsBytes, 0>>>(xw, ww, y, m, n, padded_k(k), tiles_m, tiles_n, 1, Epilogue{});
+        kern<<<(unsigned)grid, C::THREADS, kLdsBytes, 0>>>(xw, ww, y, m, n, padded_k(k), tiles_m, tiles_n, Epilogue{});
     CHECK(hipEventRecord(e1, 0));
     CHECK(hipDeviceSynchronize());
     CHECK(hipGetLastError());

@@ -506,6 +506,45 @@ def test_tiles_of_the_small_grid_form(gpu, host_threads, m, n, k, split):
     assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="mfma"), want)  # never split
 
 
+@pytest.mark.parametrize("m, n, k", [
+    (1, 1, 8), (33, 65, 72), (300, 300, 1000), (255, 1025, 136),   # 32 x 32 tiles: K of one stage and more
+    (333, 1111, 264), (250, 2000, 4104),                           # 64 x 32
+    (1000, 1111, 200), (2050, 2000, 648),                          # 64 x 64
+    (66, 60, 8192), (333, 1111, 8192), (600, 1500, 8192)])         # each of them split over K
+def test_tiles_of_the_fp6_small_grid_form(gpu, host_threads, m, n, k):
+    """Every tile of the FP6 kernel's small-grid form at its edges: rows and columns past the tile
+    and past the 256-row tiles of the converted form, fewer k-fragments than waves, all output
+    types, through the workspace (twice: the counters of the split go back to zero) and on
+    caller-owned operands, whose padding the kernel must not need."""
+    import torch
+
+    import int4linear_amd as lib
+
+    x = helpers.uniform_s4(2800 + m, m, k)
+    w = helpers.uniform_s4(2900 + n, n, k)
+    want = oracle.linear_ref(x, w, threads=host_threads)
+    xp, wp = helpers.pack_bytes(x), helpers.pack_bytes(w)
+    for rep in range(2):
+        assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="fp6"), want), rep
+    rng = np.random.default_rng(m + k)
+    bias = rng.integers(-1000, 1000, size=n, dtype=np.int32)
+    rs = rng.uniform(0.1, 2.0, size=m).astype(np.float32)
+    cs = rng.uniform(0.1, 2.0, size=n).astype(np.float32)
+    xd, wd = helpers.to_device_bytes(xp), helpers.to_device_bytes(wp)
+    bd, rd, cd = (torch.from_numpy(a).to("cuda:0") for a in (bias, rs, cs))
+    helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k, kernel="fp6")
+    xc = torch.empty(lib.fp6_operand_bytes(m, k), dtype=torch.uint8, device="cuda:0")
+    wc = torch.empty(lib.fp6_operand_bytes(n, k), dtype=torch.uint8, device="cuda:0")
+    lib.fp6_convert(xd, xc, m, k)
+    lib.fp6_convert(wd, wc, n, k)
+    y = torch.full((m, n), -1, dtype=torch.int32, device="cuda:0")
+    lib.linear_fp6_converted(xc, wc, bd, None, None, y, "s32", m, n, k)
+    assert np.array_equal(y.cpu().numpy(), oracle.epilogue(want, bias))
+    yf = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+    lib.linear_fp6_converted(xc, wc, None, rd, cd, yf, "f32", m, n, k)
+    assert np.array_equal(yf.cpu().numpy().view(np.int32), oracle.epilogue(want, None, rs, cs, f32=True).view(np.int32))
+
+
 @pytest.mark.parametrize("m, n, k", [(300, 2049, 8192), (257, 1000, 4096), (512, 1024, 14336), (300, 520, 16392),
                                      (1024, 4096, 14336)])
 def test_split_k_form_of_the_fp6_kernel(gpu, host_threads, m, n, k):
