@@ -198,7 +198,9 @@ int int4linear_release_workspace(void);
 
 /* Name of the kernel INT4LINEAR_KERNEL_AUTO would pick for a shape on the current device
  * ("simple", "mfma", "fp6", "skinny"); never NULL.  Sets the device up like a compute call
- * does; without a usable device the answer is the one that depends on the shape alone. */
+ * does; without a usable device the answer is the one that depends on the shape alone.
+ * (K % 128 != 0 with up to 64 rows of A is multiplied by a form without scratch memory that stands
+ * in for the kernel named here.) */
 const char *int4linear_kernel_for_shape(int m, int n, int k);
 
 /* Human-readable text for a status code; never NULL. */

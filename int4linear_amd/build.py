@@ -20,7 +20,7 @@ OBJ_DIR = PKG_DIR / "csrc" / "build"
 LIB_PATH = LIB_DIR / "libint4linear.so"
 
 HIP_SOURCES = ["api.hip", "kernels_simple.hip", "kernels_mfma.hip", "kernels_grid.hip", "kernels_fp6.hip", "kernels_fp6_grid.hip",
-               "kernels_skinny.hip"]
+               "kernels_skinny.hip", "kernels_skinny_any.hip"]
 CXX_SOURCES = ["packer_host.cpp"]
 
 # Packed-FP32 VALU forms are switched off for every device compile of this project.
@@ -42,6 +42,7 @@ HIP_FLAGS = [
 # arguments the ordinary way, a few tenths of a microsecond per launch).
 EXTRA_HIP_FLAGS = {
     "kernels_skinny.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
+    "kernels_skinny_any.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"],
 }
 
 

@@ -360,6 +360,14 @@ int gemm_impl(const void *a, const void *b, void *c, int m, int n, int k, int ke
         if (source == Workspace::Static && kernel == INT4LINEAR_KERNEL_SIMPLE &&
             pick_kernel(m, n, k, pd->info, SIZE_MAX) != INT4LINEAR_KERNEL_SIMPLE)
             return INT4LINEAR_ERR_SCRATCH;
+        // Few rows of A against K that fits no tile: what would go to the FP6 kernel, or, under
+        // capture or without scratch memory, to the scalar kernel, is multiplied as it lies.
+        const bool any_k_supports = (k % 128) != 0 && skinny_any_supports(m, n, k);
+        const bool any_k_preferred = any_k_supports && skinny_any_preferred(m, n, k);
+        if (kernel != INT4LINEAR_KERNEL_FP6 ? any_k_supports : any_k_preferred) {
+            const hipError_t e = launch_skinny_any(a, b, c, m, n, k, ep, pd->info, stream);
+            return e == hipSuccess ? INT4LINEAR_OK : fail_hip(e);
+        }
     } else if (kernel == INT4LINEAR_KERNEL_FP6 && source == Workspace::Internal) {
         capturing = stream_is_capturing(stream);
     }

@@ -215,6 +215,15 @@ size_t skinny_workspace_bytes(int m, int n, int k, const DeviceInfo &dev);
 hipError_t launch_skinny_ksplit(const void *a, const void *b, void *c, int m, int n, int k, void *workspace,
                                 unsigned *arrivals, const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
 
+// Weight streaming in one launch without scratch memory for any K that is a multiple of 8
+// (kernels_skinny_any.hip): M <= 64, 32 <= K < 2^17.  skinny_any_preferred: where it is faster than
+// the FP6 kernel; ..._to_basic: than kernels_skinny.hip's fallback for K that is a multiple of 128.
+bool skinny_any_supports(int m, int n, int k);
+bool skinny_any_preferred(int m, int n, int k);
+bool skinny_any_preferred_to_basic(int m, int n, int k, const DeviceInfo &dev);
+hipError_t launch_skinny_any(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
+                             hipStream_t stream);
+
 // Device packer / unpacker, utils/packer.cpp layouts.
 hipError_t launch_pack(const int *src, int *dst, int m, int n, hipStream_t stream);
 hipError_t launch_unpack(const int *src, int *dst, int m, int n, hipStream_t stream);

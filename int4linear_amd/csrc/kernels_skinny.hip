@@ -3,7 +3,7 @@
 // as skinny_ksplit_kernel the same code with K split over workgroups as well, for 33 to 64
 // rows of X against long K), skinny_stream_kernel (very many rows of W: workgroups that
 // stay on their CU) and skinny_basic_kernel (K that is not a whole number of 128-byte
-// tiles).
+// tiles; kernels_skinny_any.hip when it is long or no multiple of 128).
 //
 // The job is HBM-bound: every byte of W (N x K/2) is read exactly once and the arithmetic
 // (v_mfma_i32_16x16x64_i8 after the same 16x nibble widening as the big int8 kernel:
@@ -37,6 +37,7 @@
 // atomic operations on data, and the result does not depend on timing (integer additions
 // commute).
 #include "kernels.h"
+#include "quad_transpose.h"
 
 #include <utility>
 
@@ -146,27 +147,6 @@ __device__ __forceinline__ void load16_untracked(v4i &dst, const void *base, uns
     asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(dst) : "v"(lane_off), "s"(base), "n"(IMM) : "memory");
 }
 __device__ __forceinline__ void settle(v4i &v) { asm volatile("" : "+v"(v)); }
-
-// Transposes a 4 x 4 arrangement of 16-byte values inside every quad of lanes: on return
-// r[t] of lane j (j = lane % 4) holds what r[j] of lane t of the same quad held.  Two
-// exchange steps (lane distance 2, then 1), each a quad permutation and a select.
-__device__ __forceinline__ void quad_transpose(v4i &r0, v4i &r1, v4i &r2, v4i &r3, int lane)
-{
-    const bool up2 = (lane & 2) != 0, up1 = (lane & 1) != 0;
-    auto exchange = [](v4i &a, v4i &b, bool upper, auto ctrl) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int fa = __builtin_amdgcn_mov_dpp(a[c], decltype(ctrl)::value, 0xF, 0xF, true);
-            const int fb = __builtin_amdgcn_mov_dpp(b[c], decltype(ctrl)::value, 0xF, 0xF, true);
-            a[c] = upper ? fb : a[c];
-            b[c] = upper ? b[c] : fa;
-        }
-    };
-    exchange(r0, r2, up2, std::integral_constant<int, 0x4E>{});  // quad_perm [2,3,0,1]
-    exchange(r1, r3, up2, std::integral_constant<int, 0x4E>{});
-    exchange(r0, r1, up1, std::integral_constant<int, 0xB1>{});  // quad_perm [1,0,3,2]
-    exchange(r2, r3, up1, std::integral_constant<int, 0xB1>{});
-}
 
 // Largest workgroup a variant is launched with.  The register-X variant with many
 // fragments (2 * T * FMX of 16 bytes) and accumulators (R * FMX of 16 bytes) per lane
@@ -1439,6 +1419,8 @@ hipError_t launch_skinny(const void *a, const void *b, void *c, int m, int n, in
                          : dispatch_t<false>(pc.p, a, b, c, m, n, k, ep, stream);
     if (m > 64)
         return hipErrorInvalidConfiguration;  // skinny_supports() says no
+    if (skinny_any_preferred_to_basic(m, n, k, dev))
+        return launch_skinny_any(a, b, c, m, n, k, ep, dev, stream);
     switch ((m + 15) / 16) {
     case 1:
         return launch_basic<1>(a, b, c, m, n, k, ep, stream);

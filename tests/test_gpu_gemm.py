@@ -545,6 +545,47 @@ def test_tiles_of_the_fp6_small_grid_form(gpu, host_threads, m, n, k):
     assert np.array_equal(yf.cpu().numpy().view(np.int32), oracle.epilogue(want, None, rs, cs, f32=True).view(np.int32))
 
 
+@pytest.mark.parametrize("m, n, k", [
+    (1, 1, 32), (3, 17, 40), (16, 15, 504), (17, 33, 520), (64, 100, 8), (64, 300, 1000),  # around a row's last chunk and unit
+    (16, 4097, 1544), (31, 4100, 72), (48, 4111, 2056), (64, 4127, 200),                   # more rows of W than 16 per CU
+    (16, 40, 7176), (32, 50, 14344), (48, 60, 7176), (64, 256, 8200),                      # sixteen waves; their neighbours
+    (5, 40, 8320), (33, 4100, 8320), (64, 70, 8320)])                                        # whole 64-byte pieces, long
+def test_few_rows_against_any_k(gpu, host_threads, m, n, k):
+    """Up to 64 rows of A against K that does not split into 128-byte tiles: the automatic choice for
+    all output types, eagerly and from a graph (where no scratch memory may be used); the last row of
+    either operand ends its allocation.  By name the weight-streaming kernel refuses K % 128."""
+    import torch
+
+    import int4linear_amd as lib
+
+    x = helpers.uniform_s4(3000 + m, m, k)
+    w = helpers.uniform_s4(3100 + n, n, k)
+    want = oracle.linear_ref(x, w, threads=host_threads)
+    xp, wp = helpers.pack_bytes(x), helpers.pack_bytes(w)
+    assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="auto"), want)
+    rng = np.random.default_rng(m + k)
+    bias = rng.integers(-1000, 1000, size=n, dtype=np.int32)
+    rs = rng.uniform(0.1, 2.0, size=m).astype(np.float32)
+    cs = rng.uniform(0.1, 2.0, size=n).astype(np.float32)
+    xd, wd = helpers.to_device_bytes(xp), helpers.to_device_bytes(wp)
+    bd, rd, cd = (torch.from_numpy(a).to("cuda:0") for a in (bias, rs, cs))
+    yf = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+    lib.linear_f32(xd, wd, bd, rd, cd, yf, m, n, k)
+    assert np.array_equal(yf.cpu().numpy().view(np.int32), oracle.epilogue(want, bias, rs, cs, f32=True).view(np.int32))
+    helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k)
+    y = torch.empty((m, n), dtype=torch.int32, device="cuda:0")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        lib.linear_s32(xd, wd, bd, y, m, n, k)
+    for _ in range(2):
+        y.fill_(-1)
+        graph.replay()
+        assert np.array_equal(y.cpu().numpy(), oracle.epilogue(want, bias))
+    if k % 128:
+        with pytest.raises(lib.Int4LinearError):
+            lib.gemm_s4s4s32(xd, wd, y, m, n, k, kernel="skinny")
+
+
 @pytest.mark.parametrize("m, n, k", [(300, 2049, 8192), (257, 1000, 4096), (512, 1024, 14336), (300, 520, 16392),
                                      (1024, 4096, 14336)])
 def test_split_k_form_of_the_fp6_kernel(gpu, host_threads, m, n, k):
