@@ -78,7 +78,13 @@ __device__ __forceinline__ void dma16(const void *base, unsigned lane_off, unsig
                      : "memory");
 }
 
-// The same with the LDS address given as a wave-uniform base plus the constant LDS_OFF: one
+// Four bytes per lane straight into LDS at lds_addr + 4*lane.
+__device__ __forceinline__ void dma4(const void *base, unsigned lane_off, unsigned lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(lane_off), "s"(base), "s"(lds_addr) : "memory");
+}
+
+// dma16 with the LDS address given as a wave-uniform base plus the constant LDS_OFF: one
 // scalar addition straight into M0 instead of a precomputed address per load.
 template <bool NT, int IMM, int LDS_OFF>
 __device__ __forceinline__ void dma16_at(const void *base, unsigned lane_off, unsigned lds_base)
@@ -160,6 +166,11 @@ constexpr int max_threads(int t, int r, int fmx, bool xdma)
 // of W, row group of X).
 constexpr int head_bytes(int r, int fmx) { return r * fmx * 1024; }
 
+// LDS behind the waves' tiles, where there is room: the bias and the column scales of the
+// workgroup's (up to 64) rows of W and the row scales of its rows of X, 64 words each.
+constexpr int kEpilogueBytes = 3 * 256;
+constexpr int kEpilogueArgument = 48;  // offset of the kernels' Epilogue: behind three pointers and an aligned v4i
+
 // T tiles per wave, R row groups per workgroup, FMX 16-row groups of X (M <= 16*FMX).
 // XDMA: X tiles go through LDS like W; otherwise they are loaded into registers in
 // fragment layout (for K so long that X tiles do not fit in LDS next to the W staging).
@@ -172,23 +183,25 @@ constexpr int head_bytes(int r, int fmx) { return r * fmx * 1024; }
 // only the last group's share, the meeting and the stores are exposed after the last byte
 // arrives.
 //
+// EPILOGUE: false for plain int32 sums (a build of its own: the epilogue's code in the way of the plain
+// path cost it 0.1 us, fetched instructions that nothing overlaps).
+//
 // KSPLIT: the grid is (row blocks) x (2 or 4 slices of K, four as launched today); workgroup b takes row block
 // b / slices and slice b % slices of K (an even split into whole tiles; workgroup ids go round
 // the XCDs, so an XCD's workgroups share one or two slices of X), leaves its partial sums
 // in `partial` and counts itself in at `arrivals`; the last of a row block's workgroups to
 // arrive adds them up and stores (see the end of the function).
-template <int T, int R, int FMX, bool XDMA, bool RAGGED, bool KSPLIT>
-__device__ __forceinline__ void skinny_body(const uint8_t *X, const uint8_t *W, int32_t *Y, v4i dims, const Epilogue &ep_all,
-                                            int *partial, unsigned *arrivals)
+template <int T, int R, int FMX, bool XDMA, bool RAGGED, bool KSPLIT, bool EPILOGUE>
+__device__ __forceinline__ void skinny_body(const uint8_t *X, const uint8_t *W, int32_t *Y, v4i dims, int *partial, unsigned *arrivals)
 {
     static_assert(!(KSPLIT && RAGGED), "slices of K are whole numbers of tiles");
-    // dims: { M | passes << 8 | S << 16 | plain << 24 | log2(slices of K) << 25, N, K, rows_blk } --
+    // dims: { M | passes << 8 | S << 16 | log2(slices of K) << 25 | early << 27, N, K, rows_blk } --
     // one argument instead of seven: the host's cost of a launch grows with the number of
-    // arguments (0.1 us each), and these launches are short enough for that to show.  `plain`
-    // says that ep_all is all zero, which the storing wave then knows without loading it.
+    // arguments (0.1 us each), and these launches are short enough for that to show.  `early`
+    // says that the launch has kEpilogueBytes of LDS for the epilogue's operands.
     int M = dims[0] & 0xFF, passes = (dims[0] >> 8) & 0xFF;
     const int waves = (dims[0] >> 16) & 0xFF;
-    const bool plain = (dims[0] >> 24) & 1;
+    const bool early = EPILOGUE && (dims[0] >> 27) & 1;
     const int N = dims[1], K = dims[2], rows_blk = dims[3];
     const int kslices_log2 = KSPLIT ? (dims[0] >> 25) & 3 : 0;
     const int kslices = 1 << kslices_log2;
@@ -262,6 +275,8 @@ __device__ __forceinline__ void skinny_body(const uint8_t *X, const uint8_t *W, 
     // S * T tiles, each wave refills its own LDS tiles (nobody else reads them, and its own
     // reads of the previous pass have been consumed).
     int skip = 0;
+    Epilogue ep;
+    const int epilogue_at = kHead + waves * kWaveTiles * kTileBytes;
 #pragma unroll 1
     for (int pass = 0; pass < passes; ++pass) {
     {
@@ -354,6 +369,32 @@ __device__ __forceinline__ void skinny_body(const uint8_t *X, const uint8_t *W, 
     if constexpr (T > 1)
         issue_w(kZero, kOne, kRestOfGroup);
     static_for<kAhead>([&](auto g) { issue_w(std::integral_constant<int, decltype(g)::value + 1>{}, kZero, kAllTiles); });
+    // The epilogue's operands, behind the first loads and by one wave for all: the storing waves
+    // would otherwise meet two dependent trips to memory (the kernel arguments', the operands') at
+    // the end, where nothing overlaps them (bf16 output, us: 1 x 4096 x 4096 4.41 -> 4.11, 16 x 4096 x 4096
+    // 4.55 -> 4.24, 64 x 4096 x 4096 6.8 -> 6.35, 64 x 12288 x 1024 12.7 -> 10.6).  (The loads are younger than every load counted so
+    // far: this wave's waits for tiles last up to three loads longer than needed, and its last
+    // one, for everything, covers them.)
+    if (EPILOGUE && pass == 0) {
+        // (from the argument segment by hand: named, the argument is loaded and waited for at the
+        // top of the kernel, in front of the first loads)
+        auto arg = (const __attribute__((address_space(4))) Epilogue *)((const __attribute__((address_space(4))) uint8_t *)
+                                                                            __builtin_amdgcn_kernarg_segment_ptr() + kEpilogueArgument);
+        asm volatile("" : "+s"(arg));
+        ep.bias = arg->bias;
+        ep.row_scale = arg->row_scale;
+        ep.col_scale = arg->col_scale;
+        ep.out = arg->out;
+        if (early && wave == waves - 1) {
+            const unsigned at_n = 4 * (unsigned)min(lane_here, rows_here - 1), at_m = 4 * (unsigned)min(lane_here, M - 1);
+            if (ep.bias)
+                dma4(ep.bias + n0, at_n, lds_base + epilogue_at);
+            if (ep.col_scale)
+                dma4(ep.col_scale + n0, at_n, lds_base + epilogue_at + 256);
+            if (ep.row_scale)
+                dma4(ep.row_scale, at_m, lds_base + epilogue_at + 512);
+        }
+    }
     }
 
     // Waits until tile t of the wave's i-th row group has landed: loads complete in issue
@@ -607,52 +648,77 @@ __device__ __forceinline__ void skinny_body(const uint8_t *X, const uint8_t *W, 
                 f(0, j);
         }
     };
-    if (plain && ((N | rows_here) & 3) == 0) {
-        // Nothing to load or to convert, and a lane's four outputs exist together or not at
-        // all: the path that ends the kernel in the common case, kept to a few instructions.
+    if constexpr (!EPILOGUE) {
+        // Nothing to load or to convert: the path that ends the kernel in the commonest case, kept
+        // to a few instructions where a lane's four outputs exist together or not at all.
+        const bool together = ((N | rows_here) & 3) == 0;
         for_my_blocks([&](int i, int j) {  // block j: row group j / FMX of W, j % FMX of X
             const int rg = j / FMX, f = j % FMX;
             const v4i sum = sum_of(i, j);
-            if (f * 16 + om < M && rg * 16 + 4 * oj < rows_here)
-                *(v4i *)(Y + (size_t)(f * 16 + om) * N + n0 + rg * 16 + 4 * oj) = sum;
+            const int nb = rg * 16 + 4 * oj;  // within the workgroup's rows
+            int32_t *const y = Y + (size_t)(f * 16 + om) * N + n0 + nb;
+            if (f * 16 + om < M && nb < rows_here) {
+                if (together) {
+                    *(v4i *)y = sum;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (nb + q < rows_here)
+                            y[q] = sum[q];
+                }
+            }
         });
         return;
     }
-    // (the epilogue's operands are first looked at here, not ahead of the loads)
-    Epilogue ep = ep_all;
-    asm volatile("" : "+s"(ep.bias), "+s"(ep.row_scale), "+s"(ep.col_scale), "+s"(ep.out));
+    const int *const fetched = (const int *)(lds + epilogue_at);
     for_my_blocks([&](int i, int j) {
         const int rg = j / FMX, f = j % FMX;
         v4i sum = sum_of(i, j);
         const int m = f * 16 + om;
         const int nb = rg * 16 + 4 * oj;  // within the workgroup's rows
         if (m < M) {
-            const float rs = ep.row_scale ? ep.row_scale[m] : 1.f;
-            by_output_width(ep, [&](auto half) {
+            v4i bias = {0, 0, 0, 0}, scale = {0x3F800000, 0x3F800000, 0x3F800000, 0x3F800000};
+            int rs = 0x3F800000;
+            if (early) {
+                if (ep.bias)
+                    bias = *(const v4i *)(fetched + nb);
+                if (ep.col_scale)
+                    scale = *(const v4i *)(fetched + 64 + nb);
+                if (ep.row_scale)
+                    rs = fetched[128 + m];
+            } else {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int nn = n0 + (nb + q < rows_here ? nb + q : rows_here - 1);
-                    sum[q] = epilogue_value_of<half()>(ep, sum[q], ep.bias ? ep.bias[nn] : 0, rs, ep.col_scale ? ep.col_scale[nn] : 1.f);
+                    bias[q] = ep.bias ? ep.bias[nn] : 0;
+                    scale[q] = ep.col_scale ? __float_as_int(ep.col_scale[nn]) : 0x3F800000;
                 }
+                if (ep.row_scale)
+                    rs = __float_as_int(ep.row_scale[m]);
+            }
+            by_output_width(ep, [&](auto half) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    sum[q] = epilogue_value_of<half()>(ep, sum[q], bias[q], __int_as_float(rs), __int_as_float(scale[q]));
                 store_out4<half()>(Y, (size_t)m * N + n0 + nb, sum, rows_here - nb, nb + 3 < rows_here && ((N | n0) & 3) == 0);
             });
         }
     });
 }
 
-template <int T, int R, int FMX, bool XDMA, bool RAGGED>
+template <int T, int R, int FMX, bool XDMA, bool RAGGED, bool EPILOGUE>
 __global__ __launch_bounds__(max_threads(T, R, FMX, XDMA)) void skinny_kernel(const uint8_t *X, const uint8_t *W, int32_t *Y,
-                                                                              v4i dims, Epilogue ep_all)
+                                                                              v4i dims, Epilogue)
 {
-    skinny_body<T, R, FMX, XDMA, RAGGED, false>(X, W, Y, dims, ep_all, nullptr, nullptr);
+    skinny_body<T, R, FMX, XDMA, RAGGED, false, EPILOGUE>(X, W, Y, dims, nullptr, nullptr);
 }
 
-template <int T, int R, int FMX, bool XDMA>
+template <int T, int R, int FMX, bool XDMA, bool EPILOGUE>
 __global__ __launch_bounds__(max_threads(T, R, FMX, XDMA)) void skinny_ksplit_kernel(const uint8_t *X, const uint8_t *W, int32_t *Y,
-                                                                                     v4i dims, Epilogue ep_all, int *partial,
+                                                                                     v4i dims, Epilogue, int *partial,
                                                                                      unsigned *arrivals)
 {
-    skinny_body<T, R, FMX, XDMA, false, true>(X, W, Y, dims, ep_all, partial, arrivals);
+    skinny_body<T, R, FMX, XDMA, false, true, EPILOGUE>(X, W, Y, dims, partial, arrivals);
 }
 
 // ---- long-W form: many 16-row groups of W per CU, FMX 16-row groups of X.
@@ -1076,36 +1142,36 @@ struct KSplit {
     unsigned *arrivals = nullptr;
 };
 
-template <int T, int R, int FMX, bool XDMA>
-hipError_t launch_plan(const Plan &p, const void *a, const void *b, void *c, int m, int n, int k,
-                       const Epilogue &ep, hipStream_t stream, const KSplit &split = KSplit{})
+template <int T, int R, int FMX, bool XDMA, bool EPILOGUE>
+hipError_t launch_form(const Plan &p, const void *a, const void *b, void *c, int m, int n, int k,
+                       const Epilogue &ep, hipStream_t stream, const KSplit &split)
 {
     if constexpr (!variant_exists(T, R, FMX, XDMA)) {
         return p.s == 0 ? hipSuccess : hipErrorInvalidConfiguration;  // never planned
     } else {
+    const int early = EPILOGUE && p.lds + kEpilogueBytes <= kMaxLds;
+    const int lds = p.lds + (early ? kEpilogueBytes : 0);
     if constexpr (ksplit_variant_exists(T, R, FMX, XDMA)) {
-        auto kern = skinny_ksplit_kernel<T, R, FMX, XDMA>;
+        auto kern = skinny_ksplit_kernel<T, R, FMX, XDMA, EPILOGUE>;
         if (p.s == 0) {  // set-up call, for both forms
             const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
             if (e != hipSuccess)
                 return e;
         } else if (split.slices > 1) {
             const unsigned row_blocks = (unsigned)((n + p.rows_blk - 1) / p.rows_blk);
-            const int plain = !ep.bias && !ep.row_scale && !ep.col_scale && !ep.out;
-            kern<<<row_blocks * split.slices, p.s * 64, p.lds, stream>>>(
+            kern<<<row_blocks * split.slices, p.s * 64, lds, stream>>>(
                 (const uint8_t *)a, (const uint8_t *)b, (int32_t *)c,
-                (v4i){m | (p.passes << 8) | (p.s << 16) | (plain << 24) | ((split.slices == 4 ? 2 : 1) << 25), n, k, p.rows_blk}, ep, split.partial,
+                (v4i){m | (p.passes << 8) | (p.s << 16) | ((split.slices == 4 ? 2 : 1) << 25) | (early << 27), n, k, p.rows_blk}, ep, split.partial,
                 split.arrivals);
             return hipGetLastError();
         }
     } else if (split.slices > 1) {
         return hipErrorInvalidConfiguration;
     }
-    auto kern = p.ragged ? skinny_kernel<T, R, FMX, XDMA, true> : skinny_kernel<T, R, FMX, XDMA, false>;
+    auto kern = p.ragged ? skinny_kernel<T, R, FMX, XDMA, true, EPILOGUE> : skinny_kernel<T, R, FMX, XDMA, false, EPILOGUE>;
     if (p.s == 0)  // set-up call: raise the dynamic-LDS limit of this instantiation
         return hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
     const unsigned grid = (unsigned)((n + p.rows_blk - 1) / p.rows_blk);
-    const int plain = !ep.bias && !ep.row_scale && !ep.col_scale && !ep.out;
     // More than 16 * FMX rows of X go out in runs of that many, one launch each (the rows of
     // W are then streamed again, through the caches they were just pulled through).
     for (int m0 = 0; m0 < m; m0 += 16 * FMX) {
@@ -1113,15 +1179,28 @@ hipError_t launch_plan(const Plan &p, const void *a, const void *b, void *c, int
         if (run_ep.row_scale)
             run_ep.row_scale += m0;
         const int rows = m - m0 < 16 * FMX ? m - m0 : 16 * FMX;
-        kern<<<grid, p.s * 64, p.lds, stream>>>((const uint8_t *)a + (size_t)m0 * (size_t)(k >> 1), (const uint8_t *)b,
+        kern<<<grid, p.s * 64, lds, stream>>>((const uint8_t *)a + (size_t)m0 * (size_t)(k >> 1), (const uint8_t *)b,
                                                 (int32_t *)((uint8_t *)c + (size_t)m0 * (size_t)n * (ep.out >= kOutF16 ? 2u : 4u)),
-                                                (v4i){rows | (p.passes << 8) | (p.s << 16) | (plain << 24), n, k, p.rows_blk}, run_ep);
+                                                (v4i){rows | (p.passes << 8) | (p.s << 16) | (early << 27), n, k, p.rows_blk}, run_ep);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess)
             return e;
     }
     return hipSuccess;
     }
+}
+
+template <int T, int R, int FMX, bool XDMA>
+hipError_t launch_plan(const Plan &p, const void *a, const void *b, void *c, int m, int n, int k,
+                       const Epilogue &ep, hipStream_t stream, const KSplit &split)
+{
+    const bool plain = !ep.bias && !ep.row_scale && !ep.col_scale && !ep.out;
+    if (p.s == 0) {  // set-up call, for both builds
+        const hipError_t e = launch_form<T, R, FMX, XDMA, true>(p, a, b, c, m, n, k, ep, stream, split);
+        return e == hipSuccess ? launch_form<T, R, FMX, XDMA, false>(p, a, b, c, m, n, k, ep, stream, split) : e;
+    }
+    return plain ? launch_form<T, R, FMX, XDMA, false>(p, a, b, c, m, n, k, ep, stream, split)
+                 : launch_form<T, R, FMX, XDMA, true>(p, a, b, c, m, n, k, ep, stream, split);
 }
 
 template <int T, bool XDMA>

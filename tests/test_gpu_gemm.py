@@ -546,6 +546,39 @@ def test_tiles_of_the_fp6_small_grid_form(gpu, host_threads, m, n, k):
 
 
 @pytest.mark.parametrize("m, n, k", [
+    (1, 1, 256), (64, 14400, 4608),      # one row; eighteen tiles by 64 rows of W and of X: no LDS for the epilogue's operands
+    (3, 4100, 1024), (17, 12285, 1024), (64, 12288, 512), (33, 5000, 2816)])  # a row block's and the matrix's ragged ends
+def test_epilogue_operands_of_the_decode_kernel(gpu, host_threads, m, n, k):
+    """Bias and scales, singly and together, of the weight-streaming kernel: fetched into LDS with the
+    first loads, or late where LDS has no room; and plain sums with N no multiple of 4."""
+    import torch
+
+    import int4linear_amd as lib
+
+    x = helpers.uniform_s4(3400 + m, m, k)
+    w = helpers.uniform_s4(3500 + n, n, k)
+    want = oracle.linear_ref(x, w, threads=host_threads)
+    xd, wd = helpers.to_device_bytes(helpers.pack_bytes(x)), helpers.to_device_bytes(helpers.pack_bytes(w))
+    rng = np.random.default_rng(m + k)
+    bias = rng.integers(-1000, 1000, size=n, dtype=np.int32)
+    rs = rng.uniform(0.1, 2.0, size=m).astype(np.float32)
+    cs = rng.uniform(0.1, 2.0, size=n).astype(np.float32)
+    bd, rd, cd = (torch.from_numpy(a).to("cuda:0") for a in (bias, rs, cs))
+    y = torch.full((m, n), -1, dtype=torch.int32, device="cuda:0")
+    lib.linear_s32(xd, wd, None, y, m, n, k, kernel="skinny")
+    assert np.array_equal(y.cpu().numpy(), want)
+    lib.linear_s32(xd, wd, bd, y, m, n, k, kernel="skinny")
+    assert np.array_equal(y.cpu().numpy(), oracle.epilogue(want, bias))
+    yf = torch.empty((m, n), dtype=torch.float32, device="cuda:0")
+    for b, r, c in [(1, 1, 1), (0, 1, 0), (0, 0, 1), (0, 0, 0)]:
+        yf.fill_(float("nan"))
+        lib.linear_f32(xd, wd, bd if b else None, rd if r else None, cd if c else None, yf, m, n, k, kernel="skinny")
+        ref = oracle.epilogue(want, bias if b else None, rs if r else None, cs if c else None, f32=True)
+        assert np.array_equal(yf.cpu().numpy().view(np.int32), ref.view(np.int32)), (b, r, c)
+    helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k, kernel="skinny")
+
+
+@pytest.mark.parametrize("m, n, k", [
     (1, 1, 32), (3, 17, 40), (16, 15, 504), (17, 33, 520), (64, 100, 8), (64, 300, 1000),  # around a row's last chunk and unit
     (16, 4097, 1544), (31, 4100, 72), (48, 4111, 2056), (64, 4127, 200),                   # more rows of W than 16 per CU
     (16, 40, 7176), (32, 50, 14344), (48, 60, 7176), (64, 256, 8200),                      # sixteen waves; their neighbours
