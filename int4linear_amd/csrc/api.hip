@@ -166,7 +166,7 @@ DeviceInfo current_device_info()
 int pick_kernel(int m, int n, int k, const DeviceInfo &dev, size_t limit)
 {
     if (skinny_preferred(m, n, k, dev))
-        return INT4LINEAR_KERNEL_SKINNY;
+        return skinny_tiles_preferred(m, n, k) ? INT4LINEAR_KERNEL_MFMA : INT4LINEAR_KERNEL_SKINNY;
     if (fp6_worthwhile(m, n, k, dev, limit))
         return INT4LINEAR_KERNEL_FP6;
     if (mfma_supports(m, n, k))
@@ -344,7 +344,7 @@ int gemm_impl(const void *a, const void *b, void *c, int m, int n, int k, int ke
         kernel = pick_kernel(m, n, k, pd->info, limit);
         // A stream under capture gets the kernels that need no workspace.  Whether it is one
         // is asked only when the chosen kernel would touch the internal workspace or its
-        // ordering between streams: decode calls with up to 32 rows, a few microseconds
+        // ordering between streams: decode calls with up to 16 rows, a few microseconds
         // long, never pay for the query.
         if (source == Workspace::Internal &&
             (kernel == INT4LINEAR_KERNEL_FP6 ||

@@ -197,6 +197,8 @@ hipError_t launch_fp6_grid(const void *a_conv, const void *b_conv, void *c, int 
 // the shapes for which the automatic dispatch uses it.
 bool skinny_supports(int m, int n, int k);
 bool skinny_preferred(int m, int n, int k, const DeviceInfo &dev);
+// Among those, the shapes the automatic dispatch gives to the int8 kernel all the same.
+bool skinny_tiles_preferred(int m, int n, int k);
 hipError_t skinny_init(const DeviceInfo &dev);
 hipError_t launch_skinny(const void *a, const void *b, void *c, int m, int n, int k,
                          const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);

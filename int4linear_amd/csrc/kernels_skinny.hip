@@ -1388,6 +1388,23 @@ bool skinny_preferred(int m, int n, int k, const DeviceInfo &)
     return m <= 64 && skinny_supports(m, n, k);
 }
 
+// Where the int8 kernel's tiles are the faster form for 17 to 64 rows of X.  Measured from graphs, bf16 or
+// int32 output, this kernel / that one, us:
+//   K an odd multiple of 128 (no plan with whole 128-byte tiles): 64 x 256 x 4224 9.5 / 5.9, 64 x 4096 x 4224
+//     9.5 / 6.7, 64 x 28672 x 4224 40 / 23, 24 x 8192 x 4224 8.8 / 7.6, 24 x 28672 x 8320 43 / 36; but 64 x 512 x
+//     1152 3.6 / 4.1, 40 x 4096 x 4224 6.1 / 6.5, 24 x 1024 x 4224 5.0 / 5.9, 17 x 65536 x 1152 14.6 / 18;
+//   few tiles of K, so few waves, each with all of X to multiply: 64 x 14336 x 512 9.4 / 5.5, 64 x 12288 x 1024
+//     10.6 / 6.0, 64 x 28672 x 1024 11.2 / 11.0, 64 x 57344 x 2048 30.7 / 24.8, 40 x 14336 x 1024 7.0 / 6.2; but 64 x
+//     8192 x 2048 5.6 / 6.3, 64 x 14336 x 2048 8.6 / 8.5, 40 x 28672 x 1024 9.1 / 10.3, 24 x 28672 x 512 5.4 / 8.4.
+bool skinny_tiles_preferred(int m, int n, int k)
+{
+    if (m <= 16 || m > 64 || !mfma_supports(m, n, k))
+        return false;
+    if (k % kTileK != 0)
+        return (m > 48 && (k >= 3072 || n >= 16384)) || (n >= 8192 && k > 4096);
+    return m > 32 && n > 8192 && ((k <= 1024 && (m > 48 || n <= 16384)) || (m > 48 && n > 16384 && k <= 2048));
+}
+
 namespace {
 
 // The split over K across workgroups.  Whole rows of W per workgroup mean that every
@@ -1432,6 +1449,19 @@ bool make_ksplit_plan(int m, int n, int k, int cu_count, Plan &p, int &slices)
     return true;
 }
 
+// Where those slices are better taken by the int8 kernel's tiles, which share X among their rows of W
+// (called eagerly, bf16, us, without / with).  Where the split above does not apply: 64 x 512 x 16384 14.6 /
+// 8.3, 64 x 3584 x 18944 16.9 / 15.2, 64 x 4096 x 12288 12.8 / 12.1, 49 x 1024 x 12288 11.8 / 7.6, 40 x 1024 x 16384
+// 10.7 / 8.2, 32 x 2048 x 16384 10.1 / 8.6, 17 x 512 x 16384 8.5 / 7.8, but 17 x 2048 x 12288 7.3 / 7.9; where it
+// does, only with more than 48 rows of X: 64 x 4096 x 14336 14.3 / 13.5, but 64 x 4096 x 16384 14.2 / 15.0,
+// 64 x 4096 x 28672 20.1 / 20.4, 48 x 4096 x 14336 12.4 / 12.8.
+bool tiles_split(int m, int n, int k, bool own_split)
+{  // (m <= 64)
+    if (own_split)
+        return m > 48 && n <= 4096 && k < 16384;
+    return m > 48 ? n <= 4096 && k >= 12288 : m > 16 && n <= 2048 && k >= 16384;
+}
+
 // The plans of the shape a host thread asked for last: a decode loop calls with a handful of
 // shapes over and over, and next to a kernel of a few microseconds the plan search (some
 // hundred candidate splits) is not free.
@@ -1442,6 +1472,7 @@ struct PlanCache {
     Plan p;
     int slices = 1;  // > 1: the split over K across workgroups applies, with plan `split`
     Plan split;
+    bool tiles = false;  // split over K, but over the int8 kernel's tiles
     size_t split_bytes = 0;
 };
 thread_local PlanCache t_plan;
@@ -1453,12 +1484,18 @@ PlanCache &plans_for(int m, int n, int k, const DeviceInfo &dev)
         pc.kind = make_stream_plan(m, n, k, dev.cu_count, pc.sp) ? 1 : make_plan(m, n, k, dev.cu_count, pc.p) ? 2 : 3;
         pc.slices = 1;
         pc.split_bytes = 0;
+        pc.tiles = false;
         if (pc.kind == 2 && make_ksplit_plan(m, n, k, dev.cu_count, pc.split, pc.slices)) {
             const size_t row_blocks = (size_t)((n + pc.split.rows_blk - 1) / pc.split.rows_blk);
             pc.split_bytes = row_blocks * pc.slices * pc.split.r * pc.split.fmx * 1024;
         } else {
             pc.slices = 1;
         }
+        if (pc.kind == 2 && tiles_split(m, n, k, pc.slices > 1))
+            if (const size_t bytes = grid_split_bytes(m, n, k, dev)) {
+                pc.tiles = true;
+                pc.split_bytes = bytes;
+            }
         pc.m = m;
         pc.n = n;
         pc.k = k;
@@ -1471,7 +1508,7 @@ PlanCache &plans_for(int m, int n, int k, const DeviceInfo &dev)
 
 size_t skinny_workspace_bytes(int m, int n, int k, const DeviceInfo &dev)
 {
-    if (m <= 32 || !skinny_supports(m, n, k))  // (the common decode call: not even a look at the cache)
+    if (m <= 16 || (m <= 32 && n > 2048) || !skinny_supports(m, n, k))  // (the common decode call: not even a look at the cache)
         return 0;
     return plans_for(m, n, k, dev).split_bytes;
 }
@@ -1480,6 +1517,8 @@ hipError_t launch_skinny_ksplit(const void *a, const void *b, void *c, int m, in
                                 unsigned *arrivals, const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
 {
     PlanCache &pc = plans_for(m, n, k, dev);
+    if (pc.tiles && workspace && arrivals)
+        return launch_grid_split(a, b, c, m, n, k, workspace, arrivals, ep, dev, stream);
     if (pc.slices <= 1 || !workspace || !arrivals)
         return launch_skinny(a, b, c, m, n, k, ep, dev, stream);
     const KSplit split{pc.slices, (int *)workspace, arrivals};

@@ -578,6 +578,38 @@ def test_epilogue_operands_of_the_decode_kernel(gpu, host_threads, m, n, k):
     helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k, kernel="skinny")
 
 
+@pytest.mark.parametrize("m, n, k, kernel", [
+    (49, 130, 3200, "mfma"), (48, 130, 3200, "skinny"), (17, 8200, 4224, "mfma"), (16, 8200, 4224, "skinny"),   # odd multiples of 128
+    (33, 8193, 512, "mfma"), (32, 8193, 512, "skinny"), (64, 16400, 2048, "mfma"), (64, 16384, 2048, "skinny"),  # few tiles of K
+    (64, 520, 12288, "skinny"), (49, 4096, 14336, "skinny"), (17, 60, 16384, "skinny"), (33, 1000, 20480, "skinny")])  # slices as tiles
+def test_decode_shapes_on_either_side_of_the_tiled_form(gpu, host_threads, m, n, k, kernel):
+    """Where 17 to 64 rows of A go to the int8 kernel's tiles, and their neighbours that do not: both
+    entry points, each twice (counters of a split go back to zero), and from a graph (no workspace)."""
+    import torch
+
+    import int4linear_amd as lib
+
+    x = helpers.uniform_s4(3600 + m, m, k)
+    w = helpers.uniform_s4(3700 + n, n, k)
+    want = oracle.linear_ref(x, w, threads=host_threads)
+    assert lib.kernel_for_shape(m, n, k) == kernel
+    xd, wd = helpers.to_device_bytes(helpers.pack_bytes(x)), helpers.to_device_bytes(helpers.pack_bytes(w))
+    y = torch.empty((m, n), dtype=torch.int32, device="cuda:0")
+    for call in (lib.gemm_s4s4s32, lib.gemm_s4s4s32_static) * 2:
+        y.fill_(-1)
+        call(xd, wd, y, m, n, k)
+        assert np.array_equal(y.cpu().numpy(), want), call
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        lib.gemm_s4s4s32(xd, wd, y, m, n, k)
+    for _ in range(2):
+        y.fill_(-1)
+        graph.replay()
+        assert np.array_equal(y.cpu().numpy(), want)
+    bias, rs, cs = np.arange(n, dtype=np.int32), np.linspace(0.5, 2, m, dtype=np.float32), np.linspace(0.1, 1, n, dtype=np.float32)
+    helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k)
+
+
 @pytest.mark.parametrize("m, n, k", [
     (1, 1, 32), (3, 17, 40), (16, 15, 504), (17, 33, 520), (64, 100, 8), (64, 300, 1000),  # around a row's last chunk and unit
     (16, 4097, 1544), (31, 4100, 72), (48, 4111, 2056), (64, 4127, 200),                   # more rows of W than 16 per CU
