@@ -8,8 +8,6 @@ device memory and the stream) or raw integer device addresses.
 """
 from __future__ import annotations
 
-import ctypes
-
 import numpy as np
 
 from . import _lib
@@ -29,9 +27,14 @@ def _ptr(obj) -> int:
 
 
 def _current_stream() -> int:
+    """The handle torch.cuda.current_stream().cuda_stream gives, asked for without the Stream object that
+    call makes: 2.7 us, longer than the smallest kernels run and more than a third of a call's 7.4 us on
+    the host, against 0.3."""
     import torch
 
-    return torch.cuda.current_stream().cuda_stream
+    if not torch.cuda.is_initialized():  # (torch sets itself up, or says why it cannot)
+        return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def init() -> None:
@@ -47,7 +50,7 @@ def gemm_s4s4s32(a_packed_d, b_packed_d, c_d, m: int, n: int, k: int, *, kernel:
     if stream is None:
         stream = _current_stream()
     st = lib.int4linear_gemm_s4s4s32_ex(_ptr(a_packed_d), _ptr(b_packed_d), _ptr(c_d), m, n, k,
-                                        KERNELS[kernel], ctypes.c_void_p(stream))
+                                        KERNELS[kernel], stream)
     _lib.check(st)
 
 
@@ -61,7 +64,7 @@ def gemm_s4s4s32_static(a_packed_d, b_packed_d, c_d, m: int, n: int, k: int, *, 
     if stream is None:
         stream = _current_stream()
     _lib.check(lib.int4linear_gemm_s4s4s32_static(_ptr(a_packed_d), _ptr(b_packed_d), _ptr(c_d), m, n, k,
-                                                  ctypes.c_void_p(stream)))
+                                                  stream))
 
 
 def linear_s32(x_packed_d, w_packed_d, bias_d, y_d, m: int, n: int, k: int, *, kernel: str = "auto",
@@ -71,7 +74,7 @@ def linear_s32(x_packed_d, w_packed_d, bias_d, y_d, m: int, n: int, k: int, *, k
     if stream is None:
         stream = _current_stream()
     _lib.check(lib.int4linear_linear_s32(_ptr(x_packed_d), _ptr(w_packed_d), _ptr(bias_d), _ptr(y_d), m, n, k,
-                                         KERNELS[kernel], ctypes.c_void_p(stream)))
+                                         KERNELS[kernel], stream))
 
 
 def linear_f32(x_packed_d, w_packed_d, bias_d, row_scale_d, col_scale_d, y_d, m: int, n: int, k: int, *,
@@ -83,7 +86,7 @@ def linear_f32(x_packed_d, w_packed_d, bias_d, row_scale_d, col_scale_d, y_d, m:
         stream = _current_stream()
     _lib.check(lib.int4linear_linear_f32(_ptr(x_packed_d), _ptr(w_packed_d), _ptr(bias_d), _ptr(row_scale_d),
                                          _ptr(col_scale_d), _ptr(y_d), m, n, k, KERNELS[kernel],
-                                         ctypes.c_void_p(stream)))
+                                         stream))
 
 
 def linear_f16(x_packed_d, w_packed_d, bias_d, row_scale_d, col_scale_d, y_d, m: int, n: int, k: int, *,
@@ -94,7 +97,7 @@ def linear_f16(x_packed_d, w_packed_d, bias_d, row_scale_d, col_scale_d, y_d, m:
         stream = _current_stream()
     _lib.check(lib.int4linear_linear_f16(_ptr(x_packed_d), _ptr(w_packed_d), _ptr(bias_d), _ptr(row_scale_d),
                                          _ptr(col_scale_d), _ptr(y_d), m, n, k, KERNELS[kernel],
-                                         ctypes.c_void_p(stream)))
+                                         stream))
 
 
 def linear_bf16(x_packed_d, w_packed_d, bias_d, row_scale_d, col_scale_d, y_d, m: int, n: int, k: int, *,
@@ -105,7 +108,7 @@ def linear_bf16(x_packed_d, w_packed_d, bias_d, row_scale_d, col_scale_d, y_d, m
         stream = _current_stream()
     _lib.check(lib.int4linear_linear_bf16(_ptr(x_packed_d), _ptr(w_packed_d), _ptr(bias_d), _ptr(row_scale_d),
                                           _ptr(col_scale_d), _ptr(y_d), m, n, k, KERNELS[kernel],
-                                          ctypes.c_void_p(stream)))
+                                          stream))
 
 
 def fp6_operand_bytes(rows: int, k: int) -> int:
@@ -118,7 +121,7 @@ def fp6_convert(packed_d, converted_d, rows: int, k: int, *, stream: int | None 
     lib = _lib.load()
     if stream is None:
         stream = _current_stream()
-    _lib.check(lib.int4linear_fp6_convert(_ptr(packed_d), _ptr(converted_d), rows, k, ctypes.c_void_p(stream)))
+    _lib.check(lib.int4linear_fp6_convert(_ptr(packed_d), _ptr(converted_d), rows, k, stream))
 
 
 def gemm_fp6_converted(a_conv_d, b_conv_d, c_d, m: int, n: int, k: int, *, stream: int | None = None) -> None:
@@ -127,7 +130,7 @@ def gemm_fp6_converted(a_conv_d, b_conv_d, c_d, m: int, n: int, k: int, *, strea
     if stream is None:
         stream = _current_stream()
     _lib.check(lib.int4linear_gemm_fp6_converted(_ptr(a_conv_d), _ptr(b_conv_d), _ptr(c_d), m, n, k,
-                                                 ctypes.c_void_p(stream)))
+                                                 stream))
 
 
 OUT_TYPES = {"s32": 0, "f32": 1, "f16": 2, "bf16": 3}  # INT4LINEAR_OUT_*
@@ -142,7 +145,7 @@ def linear_fp6_converted(x_conv_d, w_conv_d, bias_d, row_scale_d, col_scale_d, y
         stream = _current_stream()
     _lib.check(lib.int4linear_linear_fp6_converted(_ptr(x_conv_d), _ptr(w_conv_d), _ptr(bias_d), _ptr(row_scale_d),
                                                    _ptr(col_scale_d), _ptr(y_d), OUT_TYPES[out_type], m, n, k,
-                                                   ctypes.c_void_p(stream)))
+                                                   stream))
 
 
 def workspace_bytes(m: int, n: int, k: int) -> int:
@@ -166,14 +169,14 @@ def pack_device(src_d, dst_d, m: int, n: int, *, stream: int | None = None) -> N
     lib = _lib.load()
     if stream is None:
         stream = _current_stream()
-    _lib.check(lib.int4linear_pack_s32_to_s4(_ptr(src_d), _ptr(dst_d), m, n, ctypes.c_void_p(stream)))
+    _lib.check(lib.int4linear_pack_s32_to_s4(_ptr(src_d), _ptr(dst_d), m, n, stream))
 
 
 def unpack_device(src_d, dst_d, m: int, n: int, *, stream: int | None = None) -> None:
     lib = _lib.load()
     if stream is None:
         stream = _current_stream()
-    _lib.check(lib.int4linear_unpack_s4_to_s32(_ptr(src_d), _ptr(dst_d), m, n, ctypes.c_void_p(stream)))
+    _lib.check(lib.int4linear_unpack_s4_to_s32(_ptr(src_d), _ptr(dst_d), m, n, stream))
 
 
 def _launch(symbol: str, x_packed_d, w_packed_d, y_d, m: int, n: int, k: int) -> None:

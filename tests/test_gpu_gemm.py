@@ -578,6 +578,24 @@ def test_epilogue_operands_of_the_decode_kernel(gpu, host_threads, m, n, k):
     helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k, kernel="skinny")
 
 
+def test_default_stream_of_a_call(gpu):
+    """Calls go to torch's current stream of the calling thread, whichever that is."""
+    import threading
+
+    import torch
+
+    from int4linear_amd import api
+
+    side, seen = torch.cuda.Stream(), []
+    assert api._current_stream() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert api._current_stream() == side.cuda_stream != torch.cuda.default_stream().cuda_stream
+        thread = threading.Thread(target=lambda: seen.append((api._current_stream(), torch.cuda.current_stream().cuda_stream)))
+        thread.start()
+        thread.join()
+    assert seen[0][0] == seen[0][1] and api._current_stream() == torch.cuda.current_stream().cuda_stream
+
+
 @pytest.mark.parametrize("m, n, k, kernel", [
     (49, 130, 3200, "mfma"), (48, 130, 3200, "skinny"), (17, 8200, 4224, "mfma"), (16, 8200, 4224, "skinny"),   # odd multiples of 128
     (33, 8193, 512, "mfma"), (32, 8193, 512, "skinny"), (64, 16400, 2048, "mfma"), (64, 16384, 2048, "skinny"),  # few tiles of K
