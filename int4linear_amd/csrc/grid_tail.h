@@ -4,6 +4,7 @@
 #pragma once
 #include "kernels.h"
 
+#include <numeric>
 #include <type_traits>
 #include <utility>
 
@@ -53,10 +54,11 @@ __device__ __forceinline__ void grid_tile_coords(int v, int total, int tiles_m, 
 template <int FM, int FN, int KG, bool HALF_OUT>
 struct GridTail {
     static constexpr int KEEP = FM * FN * 16 / KG;
-    static constexpr int FRAGS = KEEP > 16 ? KEEP / 16 : 1;  // fragments the wave's sums come from
+    static constexpr int RUN = std::gcd(KEEP, 16);  // sums in a row that are in one fragment
+    static constexpr int FRAGS = KEEP / RUN;        // such runs
     static constexpr int BM = FM * kGridFrag, BN = FN * kGridFrag;
     static constexpr int LDS_BYTES = KG * (KG - 1) * KEEP * 256;
-    static_assert(KEEP % 2 == 0 && (KEEP <= 16 ? 16 % KEEP == 0 : KEEP % 16 == 0), "parts of fragments or whole ones");
+    static_assert(KEEP % 2 == 0, "exchange() sends pairs");
 
     int lane, wave, m0, n0, M, N;
     int bias[FRAGS];
@@ -68,7 +70,7 @@ struct GridTail {
         const int r = wave * KEEP + q, t = r % 16;
         return r / 16 / FN * kGridFrag + 8 * (t / 4) + 4 * (lane >> 5) + t % 4;
     }
-    __device__ __forceinline__ int col_of(int f) const { return (wave * KEEP / 16 + f) % FN * kGridFrag + (lane & 31); }
+    __device__ __forceinline__ int col_of(int f) const { return (wave * KEEP + f * RUN) / 16 % FN * kGridFrag + (lane & 31); }
 
     // The epilogue's operands (clamped inside the matrix).  Called early, behind the first loads
     // of the main loop, so that nothing waits for them at the end.
@@ -190,13 +192,13 @@ struct GridTail {
             col_off[f] = col_of(f) < cols_left ? (unsigned)col_of(f) * kElem : 0x40000000u;
 #pragma unroll
         for (int q = 0; q < KEEP; ++q) {
-            const unsigned off = (row_of(q) < rows_left ? (unsigned)row_of(q) * (unsigned)N * kElem : 0x80000000u) + col_off[q / 16];
+            const unsigned off = (row_of(q) < rows_left ? (unsigned)row_of(q) * (unsigned)N * kElem : 0x80000000u) + col_off[q / RUN];
             if constexpr (HALF_OUT)
                 __builtin_amdgcn_raw_buffer_store_b16(
-                    (unsigned short)epilogue_value16(ep, kept[q], bias[q / 16], row_scale[q], col_scale[q / 16]), rsrc, off, 0, 0);
+                    (unsigned short)epilogue_value16(ep, kept[q], bias[q / RUN], row_scale[q], col_scale[q / RUN]), rsrc, off, 0, 0);
             else
                 __builtin_amdgcn_raw_buffer_store_b32(
-                    (unsigned)(plain ? kept[q] : epilogue_value32(ep, kept[q], bias[q / 16], row_scale[q], col_scale[q / 16])), rsrc,
+                    (unsigned)(plain ? kept[q] : epilogue_value32(ep, kept[q], bias[q / RUN], row_scale[q], col_scale[q / RUN])), rsrc,
                     off, 0, 0);
         }
     }

@@ -1,15 +1,16 @@
 // Small-grid form of the int8-MFMA GEMM: shapes whose 128 x 128 tiles would leave half of the CUs
-// idle or more.  Same arithmetic as kernels_mfma.hip (packed s4 through LDS, nibbles widened to
+// idle or more, or whose 64 x 96 tiles fit the device two to a CU.  Same arithmetic as kernels_mfma.hip (packed s4 through LDS, nibbles widened to
 // 16 times their value in int8 lanes, C = acc >> 8).
 //
 // What bounds such a grid is the time to get a CU's operands to it and the length of one
 // wave's chain of instructions: with a tile per CU nothing else runs there.  Hence
 //   * all waves of a workgroup share one tile of C and split every stage's K between them.  A wave
-//     then owns a block of C large enough (64 x 64 or 64 x 32) that a widened fragment feeds
+//     then owns a block of C large enough (64 x 96 to 64 x 32) that a widened fragment feeds
 //     several MFMAs: 6 vector operations per MFMA instead of the 12 of 32 x 32 quadrants, where
 //     the vector unit, not the matrix unit, sets the pace.  The sums meet in LDS at the end: each
 //     wave collects one part of the tile and stores it.
-//   * a stage is 512 of K: whole 128-byte lines of every row, one barrier.
+//   * a stage is 512 of K: whole 128-byte lines of every row, one barrier.  (256 of K in a ring twice as
+//     deep is slower: 128 x 14336 x 4096 13.6 instead of 12.4 us, 1000 x 3000 x 4096 20.1 instead of 18.7.)
 //   * one set of packed and of widened operands is a pipeline: the even-nibble MFMAs of a unit run
 //     while its odd nibbles are masked, its odd-nibble MFMAs while the next unit's even nibbles
 //     are shifted and masked.  No registers for a second set, so three waves fit a SIMD.
@@ -306,21 +307,30 @@ using Tile32x32 = GridTile<1, 1, 8, 4, 2>;        // 64 KiB of LDS
 using Tile64x32Short = GridTile<2, 1, 4, 3, 2>;   // 72 KiB; four waves: less to bring together at the end
 using Tile64x32Long = GridTile<2, 1, 8, 3, 4>;    // 72 KiB; eight waves
 using Tile64x64 = GridTile<2, 2, 4, 2, 2>;        // 64 KiB
+using Tile64x96 = GridTile<2, 3, 4, 2, 2>;        // 80 KiB
 
-enum class Tile { k32x32, k64x32Short, k64x32Long, k64x64 };
+enum class Tile { k32x32, k64x32Short, k64x32Long, k64x64, k64x96 };
+
+// 128 x 128 tiles on half of the CUs at most.
+bool few_tiles(int m, int n, const DeviceInfo &dev) { return grid_tiles(m, n, 128, 128) * 2 <= dev.cu_count; }
 
 // The smallest tile of which there is at most one per CU: more of the device works, and every
 // CU pulls less.  Measured (us; 32 x 32 / 64 x 32 / 64 x 64): 100 x 1000 x 2048, 128 tiles of the
 // first, 4.2 / 4.8 / 5.8; 333 x 1111 x 4096, 385 and 210: 7.4 / 6.6 / 8.2; 128 x 8192 x 4096, 512
 // and 256: 13.0 / 9.9 / 9.4.  Eight waves on a 64 x 32 tile pay from K = 2048 on (100 x 1000 x
 // 2048 4.83 / 4.82 with four / eight; 200 x 2000 x 512 3.5 / 3.9; 65 x 4096 x 4096 7.1 / 6.5).
+// Above that, 64 x 64 or 64 x 96, whichever leaves the busiest CU fewer columns; 64 x 96 if they are
+// equal (five fragments are read and widened for six MFMAs, not four for four).  64 x 64 / 64 x 96 in us:
+// 128 x 11008 x 4096, 344 and 230 tiles, 12.5 / 11.8; 1000 x 1500 x 2048, 376 and 256, 8.6 / 8.4; 128 x
+// 14336 x 4096, 448 and 300, 13.5 / 16.2; 64 x 32768 x 1024, 512 and 342, 8.0 / 9.7.
 Tile choose_tile(int m, int n, int k, const DeviceInfo &dev)
 {
     if (grid_tiles(m, n, 32, 32) <= dev.cu_count)
         return Tile::k32x32;
     if (grid_tiles(m, n, 64, 32) <= dev.cu_count)
         return k > 2048 ? Tile::k64x32Long : Tile::k64x32Short;
-    return Tile::k64x64;
+    const auto columns = [&](int bn) { return (grid_tiles(m, n, 64, bn) + dev.cu_count - 1) / dev.cu_count * bn; };
+    return columns(64) < columns(96) ? Tile::k64x64 : Tile::k64x96;
 }
 
 // The split of K over workgroups: for 64 pieces of K and more, where one slice per tile leaves
@@ -393,6 +403,8 @@ hipError_t launch(Tile tile, const void *a, const void *b, void *c, int m, int n
         return launch_tile<Tile64x32Short>(a, b, c, m, n, k, split, ep, stream);
     case Tile::k64x32Long:
         return launch_tile<Tile64x32Long>(a, b, c, m, n, k, split, ep, stream);
+    case Tile::k64x96:
+        return launch_tile<Tile64x96>(a, b, c, m, n, k, split, ep, stream);
     default:
         return launch_tile<Tile64x64>(a, b, c, m, n, k, split, ep, stream);
     }
@@ -409,10 +421,15 @@ hipError_t grid_init(const DeviceInfo &)
         e = init_tile<Tile64x32Long>();
     if (e == hipSuccess)
         e = init_tile<Tile64x64>();
+    if (e == hipSuccess)
+        e = init_tile<Tile64x96>();
     return e;
 }
 
-bool grid_preferred(int m, int n, const DeviceInfo &dev) { return grid_tiles(m, n, 128, 128) * 2 <= dev.cu_count; }
+bool grid_preferred(int m, int n, const DeviceInfo &dev) 
+{
+    return few_tiles(m, n, dev) || grid_tiles(m, n, 64, 96) <= 2l * dev.cu_count;
+}
 
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
                        hipStream_t stream)
@@ -422,7 +439,7 @@ hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int 
 
 size_t grid_split_bytes(int m, int n, int k, const DeviceInfo &dev)
 {
-    return grid_preferred(m, n, dev) ? plan_split(m, n, k, dev).bytes : 0;
+    return few_tiles(m, n, dev) ? plan_split(m, n, k, dev).bytes : 0;
 }
 
 hipError_t launch_grid_split(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,

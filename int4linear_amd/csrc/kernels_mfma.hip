@@ -1091,9 +1091,7 @@ hipError_t launch_mfma(const void *a, const void *b, void *c, int m, int n, int 
                              ((n + CfgLarge::BN - 1) / CfgLarge::BN);
     // Few 128 x 128 tiles per CU: the form whose two waves per SIMD split K.
     const int pair_m = (m + kPairTile - 1) / kPairTile, pair_n = (n + kPairTile - 1) / kPairTile;
-    // ... and so few that they would leave half of the CUs idle: smaller tiles (with more than
-    // cu_count / 2 tiles of 128 x 128 the larger tile wins: 1000 x 3000 x 4096 18.1 us, 18.9 with
-    // the small-grid form).
+    // ... and so few that smaller tiles leave the busiest CU less to do (kernels_grid.hip).
     if (grid_preferred(m, n, dev))
         return launch_grid(a, b, c, m, n, k, ep, dev, stream);
     if ((long)pair_m * pair_n <= (long)dev.cu_count * kPairRounds) {

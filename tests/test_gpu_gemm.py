@@ -472,6 +472,8 @@ def test_small_grid_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     (257, 1000, 384, False), (640, 600, 1920, False), (257, 1000, 2176, False), (639, 601, 2432, False),
     # 64 x 64 tiles
     (515, 2050, 128, False), (1025, 1000, 640, False), (1000, 1111, 1152, False),
+    # 64 x 96 tiles
+    (1030, 1930, 128, False), (2049, 1100, 1152, False), (1000, 3000, 896, False),
     # each of them split over K across workgroups, with odd numbers of pieces per slice
     (65, 200, 8448, True), (200, 700, 8960, True), (250, 2300, 12544, True), (66, 60, 8320, True)])
 def test_tiles_of_the_small_grid_form(gpu, host_threads, m, n, k, split):
