@@ -123,6 +123,22 @@ def build_library(verbose: bool = False, save_temps: bool = False) -> Path:
     return LIB_PATH
 
 
+ABLATIONS = ["fp6_ablation", "int8_ablation"]
+
+
+def build_ablation(exe: Path) -> Path:
+    """Compile the measuring harness csrc/ablation/<name of exe>.cpp, which includes a kernel source and
+    launches that kernel's template itself.  The library must be there."""
+    exe.parent.mkdir(exist_ok=True)
+    flags = [f for f in HIP_FLAGS if f != "-fPIC"]
+    _run([_hipcc(), *flags, "-x", "hip", str(CSRC / "ablation" / (exe.name + ".cpp")), "-o", str(exe), f"-L{LIB_DIR}",
+          "-lint4linear", "-Wl,-rpath,$ORIGIN/" + os.path.relpath(LIB_DIR, exe.parent)])
+    return exe
+
+
 if __name__ == "__main__":
+    if "--ablation" in sys.argv:
+        print(build_ablation(Path(sys.argv[sys.argv.index("--ablation") + 1])))
+        sys.exit(0)
     path = build_library(verbose="-v" in sys.argv, save_temps="--save-temps" in sys.argv)
     print(path)

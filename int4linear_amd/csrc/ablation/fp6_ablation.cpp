@@ -12,7 +12,8 @@
 // and one [SPREAD] line.  Run it under  rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES GRBM_GUI_ACTIVE
 // for the clock and the share of cycles the matrix pipes are busy (the kernels differ in their
 // last template argument).
-#include "../../int4linear_amd/csrc/kernels_fp6.hip"
+// It launches the kernel template itself, so it stands beside the source and changes with it.
+#include "../kernels_fp6.hip"
 
 #include <cstdio>
 #include <cstdlib>

@@ -10,7 +10,7 @@
 // Run it under  rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES GRBM_GUI_ACTIVE  for the clock and the
 // share of cycles the matrix pipes are busy (the kernels differ in their last template
 // argument).
-#include "../../int4linear_amd/csrc/kernels_mfma.hip"
+#include "../kernels_mfma.hip"
 
 #include <cstdio>
 #include <cstdlib>

@@ -240,7 +240,7 @@ struct Fp6Config {
 };
 
 // What the GEMM kernel is put together from.  The library builds WholeKernel and nothing else;
-// tests/host/fp6_ablation.cpp, which compiles this file again, passes variations of its own
+// ablation/fp6_ablation.cpp, which compiles this file again, passes variations of its own
 // (derived from this one, with single members changed) to time what each part costs.
 struct WholeKernel {
     static constexpr bool kStores = true;    // a finished tile is stored

@@ -134,7 +134,7 @@ __device__ __forceinline__ void tile_coords(int v, int total, int tiles_m, int t
 }
 
 // What mfma_gemm_kernel is put together from.  The library builds WholeInt8Kernel and nothing
-// else; tests/host/int8_ablation.cpp, which compiles this file again, passes variations of
+// else; ablation/int8_ablation.cpp, which compiles this file again, passes variations of
 // its own (derived from this one, with single members changed) to time what each part costs.
 struct WholeInt8Kernel {
     static constexpr bool kStores = true;    // a finished tile is stored

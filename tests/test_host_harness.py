@@ -25,6 +25,16 @@ def test_harness_binaries_link_against_the_library():
         assert "libint4linear.so" in out and "not found" not in out, out
 
 
+def test_harnesses_here_know_the_public_interface_only():
+    """The library can change a kernel's arguments without a change to this folder: what includes kernel
+    sources stands beside them."""
+    sources = sorted(HOST.glob("*.cpp")) + sorted(HOST.glob("*.h"))
+    assert len(sources) >= 6
+    for source in sources:
+        includes = re.findall(r'#include "(.*)"', source.read_text())
+        assert set(includes) <= {"int4linear.h", "harness_common.h"}, (source, includes)
+
+
 def test_harness_usage_errors_without_a_device():
     r = subprocess.run([str(_binary("correctness")), "--entry", "v99", "16x16x128"], capture_output=True, text=True)
     assert r.returncode == 2
