@@ -109,9 +109,9 @@ int int4linear_gemm_s4s4s32(const void *a_packed_d, const void *b_packed_d, void
  * call allocates and frees nothing, records no events and takes no locks.  A shape whose
  * kernel would need more scratch than the array holds (at M = N = K the FP6 form fits up to
  * 9216) runs on the kernels that need none, as it does under graph capture through the
- * ordinary entry point; only when that would leave a large problem to the scalar kernel (K
- * not a multiple of 128, which among the fast kernels only the FP6 one takes) is the call
- * refused with INT4LINEAR_ERR_SCRATCH before anything is enqueued.  Set the device up
+ * ordinary entry point; only when that would leave a large problem to the scalar kernel (more
+ * than 64 rows of A with K not a multiple of 128, which among the fast kernels only the FP6 one
+ * takes) is the call refused with INT4LINEAR_ERR_SCRATCH before anything is enqueued.  Set the device up
  * (int4linear_init) before capturing.  All calls on one device share the one array and nothing orders
  * them: calls whose execution may overlap on a device (different streams, graphs replayed
  * concurrently) race on it; calls on one stream are ordered by the stream. */
@@ -186,7 +186,9 @@ int int4linear_linear_fp6_converted(const void *x_conv_d, const void *w_conv_d, 
 
 /* Bytes of internal workspace INT4LINEAR_KERNEL_AUTO would use for a shape on the current
  * device (0 when the chosen kernel needs none).  Sets the device up if that has not
- * happened yet, so the answer does not depend on what was called before. */
+ * happened yet, so the answer does not depend on what was called before.  It is that of the kernel
+ * which int4linear_kernel_for_shape names: an upper bound where K % 128 != 0 with up to 64 rows of
+ * A, for which the form that stands in for that kernel uses none. */
 size_t int4linear_workspace_bytes(int m, int n, int k);
 
 /* Upper bound for the internal workspace (default 1 GiB).  Shapes that would need more,

@@ -338,10 +338,19 @@ int gemm_impl(const void *a, const void *b, void *c, int m, int n, int k, int ke
     }
 
     const bool automatic = kernel == INT4LINEAR_KERNEL_AUTO;
+    // Few rows of A against K that fits no tile: what would go to the FP6 kernel or, under capture or
+    // without scratch memory, to the scalar kernel, is multiplied as it lies.
+    const bool any_k = automatic && (k % 128) != 0 && skinny_any_supports(m, n, k);
+    const auto run_any_k = [&] {
+        const hipError_t e = launch_skinny_any(a, b, c, m, n, k, ep, pd->info, stream);
+        return e == hipSuccess ? INT4LINEAR_OK : fail_hip(e);
+    };
     bool capturing = false;
     if (automatic) {
         const size_t limit = source == Workspace::Static ? kStaticScratchBytes : g_workspace_limit.load();
         kernel = pick_kernel(m, n, k, pd->info, limit);
+        if (any_k && (kernel != INT4LINEAR_KERNEL_FP6 || skinny_any_preferred(m, n, k)))
+            return run_any_k();
         // A stream under capture gets the kernels that need no workspace.  Whether it is one
         // is asked only when the chosen kernel would touch the internal workspace or its
         // ordering between streams: decode calls with up to 16 rows, a few microseconds
@@ -353,6 +362,8 @@ int gemm_impl(const void *a, const void *b, void *c, int m, int n, int k, int ke
             capturing = stream_is_capturing(stream);
             if (capturing)
                 kernel = pick_kernel(m, n, k, pd->info, 0);
+            if (any_k && kernel != INT4LINEAR_KERNEL_FP6)
+                return run_any_k();
         }
         // The static entry point falls back to the kernels without scratch memory when the
         // array is too small; it refuses only what would then be left to the scalar kernel
@@ -360,14 +371,6 @@ int gemm_impl(const void *a, const void *b, void *c, int m, int n, int k, int ke
         if (source == Workspace::Static && kernel == INT4LINEAR_KERNEL_SIMPLE &&
             pick_kernel(m, n, k, pd->info, SIZE_MAX) != INT4LINEAR_KERNEL_SIMPLE)
             return INT4LINEAR_ERR_SCRATCH;
-        // Few rows of A against K that fits no tile: what would go to the FP6 kernel, or, under
-        // capture or without scratch memory, to the scalar kernel, is multiplied as it lies.
-        const bool any_k_supports = (k % 128) != 0 && skinny_any_supports(m, n, k);
-        const bool any_k_preferred = any_k_supports && skinny_any_preferred(m, n, k);
-        if (kernel != INT4LINEAR_KERNEL_FP6 ? any_k_supports : any_k_preferred) {
-            const hipError_t e = launch_skinny_any(a, b, c, m, n, k, ep, pd->info, stream);
-            return e == hipSuccess ? INT4LINEAR_OK : fail_hip(e);
-        }
     } else if (kernel == INT4LINEAR_KERNEL_FP6 && source == Workspace::Internal) {
         capturing = stream_is_capturing(stream);
     }
@@ -379,6 +382,8 @@ int gemm_impl(const void *a, const void *b, void *c, int m, int n, int k, int ke
         // that needs none.
         if (st6 == INT4LINEAR_OK || !automatic || source == Workspace::Static)
             return st6;
+        if (any_k)
+            return run_any_k();
         kernel = mfma_supports(m, n, k) ? INT4LINEAR_KERNEL_MFMA : INT4LINEAR_KERNEL_SIMPLE;
     }
 

@@ -116,6 +116,19 @@ def test_static_falls_back_or_rejects_oversize(gpu):
         lib.gemm_s4s4s32_static(xd, wd, yd, m, n, k)
 
 
+@pytest.mark.parametrize("m, n, k", [(16, 28672, 8200), (64, 20000, 9000)])
+def test_static_takes_few_rows_with_ragged_k_of_any_size(gpu, m, n, k):
+    """K not a multiple of 128 with up to 64 rows of A needs no scratch memory, so operands whose
+    converted form would not fit the array are no reason to refuse the call."""
+    import torch
+
+    import int4linear_amd as lib
+
+    assert lib.fp6_operand_bytes(m, k) + lib.fp6_operand_bytes(n, k) > lib.api.STATIC_SCRATCH_BYTES
+    got, want = _run_pair(lib, torch, m, n, k, seed=9)
+    assert not bool((want == POISON).any()) and torch.equal(got, want)
+
+
 def test_static_entry_in_a_graph(gpu):
     """What the entry point is for: captured in a HIP graph and replayed three times with new
     operand contents and eager work between the replays, each replay checked against the
