@@ -39,6 +39,10 @@
 #include "kernels.h"
 #include "quad_transpose.h"
 
+#include <stddef.h>
+
+#include <algorithm>
+#include <type_traits>
 #include <utility>
 
 namespace int4linear {
@@ -169,7 +173,19 @@ constexpr int head_bytes(int r, int fmx) { return r * fmx * 1024; }
 // LDS behind the waves' tiles, where there is room: the bias and the column scales of the
 // workgroup's (up to 64) rows of W and the row scales of its rows of X, 64 words each.
 constexpr int kEpilogueBytes = 3 * 256;
-constexpr int kEpilogueArgument = 48;  // offset of the kernels' Epilogue: behind three pointers and an aligned v4i
+
+// The leading parameters of skinny_kernel and skinny_ksplit_kernel as they lie in the argument segment:
+// skinny_body reads the Epilogue from there by its offset.
+struct SkinnyArguments {
+    const uint8_t *X, *W;
+    int32_t *Y;
+    v4i dims;
+    Epilogue ep;
+};
+constexpr int kEpilogueArgument = offsetof(SkinnyArguments, ep);
+template <class... Rest>
+std::true_type takes_skinny_arguments(void (*)(const uint8_t *, const uint8_t *, int32_t *, v4i, Epilogue, Rest...));
+std::false_type takes_skinny_arguments(...);
 
 // T tiles per wave, R row groups per workgroup, FMX 16-row groups of X (M <= 16*FMX).
 // XDMA: X tiles go through LDS like W; otherwise they are loaded into registers in
@@ -720,6 +736,9 @@ __global__ __launch_bounds__(max_threads(T, R, FMX, XDMA)) void skinny_ksplit_ke
 {
     skinny_body<T, R, FMX, XDMA, false, true, EPILOGUE>(X, W, Y, dims, partial, arrivals);
 }
+
+static_assert(decltype(takes_skinny_arguments(skinny_kernel<1, 1, 1, true, false, true>))::value, "see SkinnyArguments");
+static_assert(decltype(takes_skinny_arguments(skinny_ksplit_kernel<2, 2, 3, true, true>))::value, "see SkinnyArguments");
 
 // ---- long-W form: many 16-row groups of W per CU, FMX 16-row groups of X.
 //
