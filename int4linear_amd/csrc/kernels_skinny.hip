@@ -1071,6 +1071,7 @@ struct Plan {
     bool xdma = true;
     bool ragged = false;  // S * T * passes > K's tiles: the last slices are partly or wholly empty
     int lds = 0;
+    int cus = 1;  // of the device
 };
 
 // Which (T, R, FMX, XDMA) combinations exist as kernels: the register-X variant holds
@@ -1138,6 +1139,7 @@ bool make_plan(int m, int n, int k, int cu_count, bool ragged, Plan &p)
     if (!fit(tiles, fmx, r, ragged, p))  // r <= rmax, so this succeeds
         return false;
     p.rows_blk = rows_blk;
+    p.cus = (int)cus;
     return true;
 }
 
@@ -1161,6 +1163,20 @@ struct KSplit {
     unsigned *arrivals = nullptr;
 };
 
+// Whether the epilogue's operands get LDS: not where the CU would then hold fewer workgroups than it
+// has to run (a set-up call counts as none).  bf16 with bias, us, without that LDS / with: 32 x 28672 x 1536, two
+// workgroups of 80 KiB a CU or one, 8.0 / 9.75; 17 x 16640 x 1536 6.9 / 8.9; 40 x 65536 x 512, four or three,
+// 16.3 / 20.1.
+bool early_epilogue(const Plan &p, int n, int slices)
+{
+    constexpr int kMaxWaves = 32;  // of a CU
+    if (p.s == 0 || p.lds + kEpilogueBytes > kMaxLds)
+        return false;
+    const long workgroups = (long)((n + p.rows_blk - 1) / p.rows_blk) * slices;
+    const long wanted = std::min((long)(kMaxWaves / p.s), (workgroups + p.cus - 1) / p.cus);
+    return kMaxLds / (p.lds + kEpilogueBytes) >= std::min(wanted, (long)(kMaxLds / p.lds));
+}
+
 template <int T, int R, int FMX, bool XDMA, bool EPILOGUE>
 hipError_t launch_form(const Plan &p, const void *a, const void *b, void *c, int m, int n, int k,
                        const Epilogue &ep, hipStream_t stream, const KSplit &split)
@@ -1168,7 +1184,7 @@ hipError_t launch_form(const Plan &p, const void *a, const void *b, void *c, int
     if constexpr (!variant_exists(T, R, FMX, XDMA)) {
         return p.s == 0 ? hipSuccess : hipErrorInvalidConfiguration;  // never planned
     } else {
-    const int early = EPILOGUE && p.lds + kEpilogueBytes <= kMaxLds;
+    const int early = EPILOGUE && early_epilogue(p, n, split.slices);
     const int lds = p.lds + (early ? kEpilogueBytes : 0);
     if constexpr (ksplit_variant_exists(T, R, FMX, XDMA)) {
         auto kern = skinny_ksplit_kernel<T, R, FMX, XDMA, EPILOGUE>;
@@ -1464,6 +1480,7 @@ bool make_ksplit_plan(int m, int n, int k, int cu_count, Plan &p, int &slices)
     if (p.s < 4 || row_blocks * p.s > kSkinnyArrivalWords)
         return false;
     p.rows_blk = rows_blk;
+    p.cus = cu_count;
     slices = kSlices;
     return true;
 }
