@@ -162,6 +162,7 @@ bool grid_preferred(int m, int n, const DeviceInfo &dev);
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
                        hipStream_t stream);
 size_t grid_split_bytes(int m, int n, int k, const DeviceInfo &dev);
+int grid_split_slices(int m, int n, int k, const DeviceInfo &dev);  // 1 = not split
 hipError_t launch_grid_split(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
                              const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
 

@@ -442,6 +442,11 @@ size_t grid_split_bytes(int m, int n, int k, const DeviceInfo &dev)
     return few_tiles(m, n, dev) ? plan_split(m, n, k, dev).bytes : 0;
 }
 
+int grid_split_slices(int m, int n, int k, const DeviceInfo &dev)
+{
+    return few_tiles(m, n, dev) ? plan_split(m, n, k, dev).slices : 1;
+}
+
 hipError_t launch_grid_split(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
                              const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
 {

@@ -1485,17 +1485,25 @@ bool make_ksplit_plan(int m, int n, int k, int cu_count, Plan &p, int &slices)
     return true;
 }
 
-// Where those slices are better taken by the int8 kernel's tiles, which share X among their rows of W
-// (called eagerly, bf16, us, without / with).  Where the split above does not apply: 64 x 512 x 16384 14.6 /
-// 8.3, 64 x 3584 x 18944 16.9 / 15.2, 64 x 4096 x 12288 12.8 / 12.1, 49 x 1024 x 12288 11.8 / 7.6, 40 x 1024 x 16384
-// 10.7 / 8.2, 32 x 2048 x 16384 10.1 / 8.6, 17 x 512 x 16384 8.5 / 7.8, but 17 x 2048 x 12288 7.3 / 7.9; where it
-// does, only with more than 48 rows of X: 64 x 4096 x 14336 14.3 / 13.5, but 64 x 4096 x 16384 14.2 / 15.0,
-// 64 x 4096 x 28672 20.1 / 20.4, 48 x 4096 x 14336 12.4 / 12.8.
-bool tiles_split(int m, int n, int k, bool own_split)
+// Where those slices are better taken by the int8 kernel's tiles, `slices` of them, which share X among
+// their rows of W.  Measured on weights that come from HBM (sets of over 768 MiB in rotation), int32, us, without /
+// with.  Where the split above does not apply: 64 x 512 x 16384 14.0 / 8.1, 64 x 4096 x 12288 11.9 / 11.2, 49 x 1024 x
+// 12288 10.9 / 7.5, 40 x 1024 x 16384 10.0 / 8.0, 32 x 2048 x 16384 9.2 / 8.3, but 32 x 2048 x 16640 in two slices 9.6 /
+// 10.7; least with a last stage of one piece per slice, 64 x 4096 x 13568 12.8 / 13.2 (from the caches 11.5 / 10.6).
+// Where it does, only with more than 48 rows of X, and with more than 3072 rows of W only up to K =
+// 16384 (the same with rotating outputs in parentheses): 64 x 2048 x 28672 13.4 / 12.8 (13.5 / 13.4), 64 x 3072 x 14336
+// 12.6 / 11.7 (12.6 / 11.9), 64 x 3072 x 16384 13.0 / 12.6 (13.0 / 12.9), 64 x 3072 x 24576 17.2 / 16.4 (17.2 / 16.8), 64 x
+// 4096 x 14336 13.2 / 12.4 (13.2 / 13.2; from the caches 12.4 / 10.9), but 64 x 4096 x 16384 13.9 / 13.2 (13.9 / 14.4), 64 x
+// 4096 x 28672 19.8 / 19.7 (20.0 / 21.4), 40 x 4096 x 14336 11.3 / 12.1, 40 x 2048 x 14336 8.6 / 9.3.
+bool tiles_split(int m, int n, int k, bool own_split, int slices)
 {  // (m <= 64)
+    if (m <= 16 || slices <= 1)
+        return false;
+    if (m <= 48)
+        return !own_split && n <= 2048 && k >= 16384 && (n <= 1024 || slices >= 4);
     if (own_split)
-        return m > 48 && n <= 4096 && k < 16384;
-    return m > 48 ? n <= 4096 && k >= 12288 : m > 16 && n <= 2048 && k >= 16384;
+        return n <= 3072 || (n <= 4096 && k < 16384);
+    return n <= 4096 && k >= 12288;
 }
 
 // The plans of the shape a host thread asked for last: a decode loop calls with a handful of
@@ -1527,11 +1535,10 @@ PlanCache &plans_for(int m, int n, int k, const DeviceInfo &dev)
         } else {
             pc.slices = 1;
         }
-        if (pc.kind == 2 && tiles_split(m, n, k, pc.slices > 1))
-            if (const size_t bytes = grid_split_bytes(m, n, k, dev)) {
-                pc.tiles = true;
-                pc.split_bytes = bytes;
-            }
+        if (pc.kind == 2 && tiles_split(m, n, k, pc.slices > 1, grid_split_slices(m, n, k, dev))) {
+            pc.tiles = true;
+            pc.split_bytes = grid_split_bytes(m, n, k, dev);
+        }
         pc.m = m;
         pc.n = n;
         pc.k = k;

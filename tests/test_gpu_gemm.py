@@ -603,7 +603,8 @@ def test_default_stream_of_a_call(gpu):
 @pytest.mark.parametrize("m, n, k, kernel", [
     (49, 130, 3200, "mfma"), (48, 130, 3200, "skinny"), (17, 8200, 4224, "mfma"), (16, 8200, 4224, "skinny"),   # odd multiples of 128
     (33, 8193, 512, "mfma"), (32, 8193, 512, "skinny"), (64, 16400, 2048, "mfma"), (64, 16384, 2048, "skinny"),  # few tiles of K
-    (64, 520, 12288, "skinny"), (49, 4096, 14336, "skinny"), (17, 60, 16384, "skinny"), (33, 1000, 20480, "skinny")])  # slices as tiles
+    (64, 520, 12288, "skinny"), (49, 4096, 14336, "skinny"), (17, 60, 16384, "skinny"), (33, 1000, 20480, "skinny"),  # slices as tiles
+    (64, 3072, 16384, "skinny"), (64, 3080, 16384, "skinny"), (33, 2048, 16640, "skinny"), (20, 1025, 16640, "skinny")])
 def test_decode_shapes_on_either_side_of_the_tiled_form(gpu, host_threads, m, n, k, kernel):
     """Where 17 to 64 rows of A go to the int8 kernel's tiles, and their neighbours that do not: both
     entry points, each twice (counters of a split go back to zero), and from a graph (no workspace)."""
@@ -630,6 +631,25 @@ def test_decode_shapes_on_either_side_of_the_tiled_form(gpu, host_threads, m, n,
         assert np.array_equal(y.cpu().numpy(), want)
     bias, rs, cs = np.arange(n, dtype=np.int32), np.linspace(0.5, 2, m, dtype=np.float32), np.linspace(0.1, 1, n, dtype=np.float32)
     helpers.check_half_width_outputs(xd, wd, want, bias, rs, cs, m, n, k)
+
+
+def test_slices_of_k_as_tiles_at_every_k(gpu):
+    """49 to 64 rows of A, K in four equal slices: the int8 kernel's tiles (two slices here) up to 3072
+    rows of W whatever K is, up to 4096 below K = 16384, else the decode kernel's own four slices; fewer
+    rows of A, or more of W than 1024 in two slices only, never.  Told apart by the partial sums' bytes."""
+    import torch
+
+    import int4linear_amd as lib
+
+    lib.init()
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes below are those of 256 compute units")
+    tile = 64 * 32 * 4
+    for n, k in ((3072, 14336), (3072, 16384), (3072, 28672), (4096, 14336)):
+        assert lib.workspace_bytes(64, n, k) == n // 32 * 2 * tile, (n, k)
+    for n, k in ((4096, 16384), (4096, 28672)):
+        assert lib.workspace_bytes(64, n, k) == n * 4 * 64 * 4, (n, k)
+    assert lib.workspace_bytes(32, 2048, 16384) > 0 and lib.workspace_bytes(32, 2048, 16640) == 0
 
 
 @pytest.mark.parametrize("m, n, k", [
