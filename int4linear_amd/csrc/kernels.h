@@ -153,12 +153,12 @@ hipError_t launch_mfma_splitk(const void *a, const void *b, void *c, int m, int 
                               const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
 
 // Its small-grid form (kernels_grid.hip), for shapes with at most half as many 128 x 128 tiles as
-// CUs or at most two 64 x 96 tiles per CU (grid_preferred).  With few tiles and long K it is split over K
-// across workgroups:
+// CUs or at most two 64 x 96 tiles per CU, and K long enough for the larger of its tiles
+// (grid_preferred).  With few tiles and long K it is split over K across workgroups:
 // grid_split_bytes() bytes of partial sums in `workspace` (8-byte aligned; 0 = the shape is not
 // split), arrivals counted at `arrivals` as by launch_skinny_ksplit below.
 hipError_t grid_init(const DeviceInfo &dev);
-bool grid_preferred(int m, int n, const DeviceInfo &dev);
+bool grid_preferred(int m, int n, int k, const DeviceInfo &dev);
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
                        hipStream_t stream);
 size_t grid_split_bytes(int m, int n, int k, const DeviceInfo &dev);

@@ -1,6 +1,7 @@
 // Small-grid form of the int8-MFMA GEMM: shapes whose 128 x 128 tiles would leave half of the CUs
-// idle or more, or whose 64 x 96 tiles fit the device two to a CU.  Same arithmetic as kernels_mfma.hip (packed s4 through LDS, nibbles widened to
-// 16 times their value in int8 lanes, C = acc >> 8).
+// idle or more, or whose 64 x 96 tiles fit the device two to a CU, with K long enough for the larger
+// tiles.  Same arithmetic as kernels_mfma.hip (packed s4 through LDS, nibbles widened to 16 times
+// their value in int8 lanes, C = acc >> 8).
 //
 // What bounds such a grid is the time to get a CU's operands to it and the length of one
 // wave's chain of instructions: with a tile per CU nothing else runs there.  Hence
@@ -333,6 +334,18 @@ Tile choose_tile(int m, int n, int k, const DeviceInfo &dev)
     return columns(64) < columns(96) ? Tile::k64x64 : Tile::k64x96;
 }
 
+// K from which the 64 x 64 and 64 x 96 tiles pay: `from`, or 1024 if every stage is full (a last stage of one
+// piece takes the time of four).  int32, us, the other form / this one, up to 128 tiles of 128 x 128:
+// 1024 x 1024 x 512 4.35 / 4.5, x 1024 5.15 / 5.15, x 1152 5.4 / 5.7, x 1408 5.8 / 5.75, x 1920 6.5 / 6.3; 1000 x 1500 x
+// 640 6.1 / 6.6, x 1024 7.0 / 6.7, x 1152 7.2 / 7.4, x 1408 7.8 / 7.5; beyond: 1000 x 3000 x 512 7.9 / 7.9, x 1024 9.4 / 9.0,
+// x 1152 9.5 / 10.6, x 2176 12.6 / 14.3, x 2560 14.1 / 13.8, x 2688 14.2 / 15.0, x 3200 15.8 / 16.3, x 3328 16.3 / 16.2,
+// x 4096 18.6 / 18.0; 2048 x 1280 x 1664 10.6 / 12.1, x 2048 11.9 / 11.6, x 2304 12.7 / 13.0, x 2816 14.0 / 14.0.
+bool long_enough(int k, int from)
+{
+    constexpr int kStageK = Tile64x96::PIECES * kPieceK;
+    return k >= from || (k >= 1024 && k % kStageK == 0);
+}
+
 // The split of K over workgroups: for 64 pieces of K and more, where one slice per tile leaves
 // CUs without work (32 x 32 and 64 x 32 tiles) or, with 64 x 64 tiles, a second workgroup fits every
 // CU.  The exchange costs some 2 us.  Measured, unsplit -> split: 200 x 136 x 16384 12.6 -> 7.9 us,
@@ -426,9 +439,17 @@ hipError_t grid_init(const DeviceInfo &)
     return e;
 }
 
-bool grid_preferred(int m, int n, const DeviceInfo &dev) 
+// 64 x 32 and 32 x 32 tiles always.  The larger ones once K is long enough: up to 128 tiles of 128 x 128
+// mfma_pair64_kernel is the other choice, beyond mfma_pair_kernel, whose tiles must not pad a quarter
+// more for K to decide (130 x 8500, 134 tiles against 267: 1024 8.8 / 6.6 us with bf16 output).
+bool grid_preferred(int m, int n, int k, const DeviceInfo &dev)
 {
-    return few_tiles(m, n, dev) || grid_tiles(m, n, 64, 96) <= 2l * dev.cu_count;
+    if (few_tiles(m, n, dev)) {
+        const Tile tile = choose_tile(m, n, k, dev);
+        return (tile != Tile::k64x64 && tile != Tile::k64x96) || long_enough(k, 1408);
+    }
+    const long tiles = grid_tiles(m, n, 64, 96);
+    return tiles <= 2l * dev.cu_count && (tiles * (64 * 96) * 5 <= grid_tiles(m, n, 128, 128) * (128 * 128) * 4 || long_enough(k, k % 512 == 128 ? 3328 : 2816));
 }
 
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,

@@ -24,10 +24,10 @@
 // tiles, and the load ring runs NSTAGE-1 stages ahead of the math ACROSS tile
 // boundaries, so the next tile's first stages are in flight while this tile stores C.
 //
-// Grids of few tiles run in a second form (mfma_pair_kernel: one 128 x 128 tile per workgroup,
-// eight waves of which the two on a SIMD split every stage's K), described where it is
-// defined, still smaller ones in that of kernels_grid.hip; shapes with few tiles and long K
-// are split over K.
+// Grids of few tiles run in a second form (mfma_pair_kernel, mfma_pair64_kernel: one 128 x 128 or
+// 64 x 64 tile per workgroup, eight waves of which the two on a SIMD split every stage's K),
+// described where it is defined, or, with K long enough, in that of kernels_grid.hip; shapes with
+// few tiles and long K are split over K.
 #include "kernels.h"
 
 #include <type_traits>
@@ -953,6 +953,149 @@ __global__ __launch_bounds__(512, DEEP ? 2 : 4) void mfma_pair_kernel(const uint
     }
 }
 
+// The same form with a 64 x 64 tile, for grids so small that 128 x 128 tiles would leave
+// most CUs without one and K so short that the form of kernels_grid.hip, whose stages are 512 of K
+// and whose sums meet four deep, has hardly started when it ends (int32, us, this form / that one: 1024 x 1024 x
+// 128 3.8 / 4.4, x 256 4.0 / 4.4, x 640 4.6 / 5.1, x 1152 5.4 / 5.7; see long_enough there): wave w and
+// wave w ^ 4 own the 32 x 32 quadrant w % 4 (one accumulator fragment) and split every stage's K; a
+// stage is 8 KiB, moved by one load per wave (waves 0..3 the four chunks of X rows, waves 4..7
+// those of W rows).
+constexpr int kTinyTile = 64;
+constexpr int kTinyStageBytes = 2 * kTinyTile * kRowBytes;    // 8 KiB
+constexpr int kTinyLdsBytes = kPairStages * kTinyStageBytes;  // 32 KiB; the merge takes 16 KiB of it
+
+template <bool HALF_OUT = false>
+__global__ __launch_bounds__(512) void mfma_pair64_kernel(const uint8_t *__restrict__ X,
+                                                          const uint8_t *__restrict__ W,
+                                                          int32_t *__restrict__ Y, int M, int N, int K,
+                                                          int tiles_m, int tiles_n, Epilogue ep)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = wave >> 2;  // which half of every stage's K; also: 0 loads X, 1 loads W
+    const int quad = wave & 3;
+    const int wm = quad >> 1, wn = quad & 1;
+    const int rowbytes = K >> 1;
+    const int KT = K / kStageK;
+    int tm, tn;
+    tile_coords(blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * kTinyTile, n0 = tn * kTinyTile;
+
+    // ---- loads: lane p of a chunk lands at byte 16 p: row p / 4, slot p % 4, and fetches the
+    //      row's chunk slot ^ swz(row).  Rows past the matrix re-read its last row.
+    const int ld_row = lane >> 2;
+    const int ld_c = (lane & 3) ^ swz(ld_row);
+    const int row_here = quad * kChunkRows + ld_row;
+    const int row = half ? min(row_here, N - 1 - n0) : min(row_here, M - 1 - m0);
+    const unsigned voff = (unsigned)row * (unsigned)rowbytes + (unsigned)ld_c * 16u;
+    const uint8_t *src_base = half ? W + (size_t)n0 * rowbytes : X + (size_t)m0 * rowbytes;
+    const unsigned lds_base = (unsigned)(size_t)I4L_LDS(lds);
+    const unsigned place = lds_base + (unsigned)(half * kTinyTile * kRowBytes + quad * kChunkBytes);
+    auto issue = [&](int st) {  // past the last stage the last one again, into a buffer nobody reads
+        const int src = st < KT ? st : KT - 1;
+        dma16(src_base + (size_t)src * kRowBytes, voff, place, (unsigned)((st % kPairStages) * kTinyStageBytes));
+    };
+#pragma unroll
+    for (int st = 0; st < kPairStages - 1; ++st)
+        issue(st);
+
+    const int fr = lane & 31;
+    const int fg = lane >> 5;
+    const unsigned rd_off = (unsigned)fr * kRowBytes + (unsigned)(((2 * half + fg) ^ swz(fr)) * 16);
+    const unsigned x_rd = (unsigned)(wm * kFrag * kRowBytes) + rd_off;
+    const unsigned w_rd = (unsigned)((kTinyTile + wn * kFrag) * kRowBytes) + rd_off;
+    const int himask = (int)0xF0F0F0F0u;
+    v16i acc;
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+        acc[t] = 0;
+    v4i xlo, xhi, wlo, whi;
+#pragma unroll 1
+    for (int st = 0; st < KT; ++st) {
+        // this wave's load of stage st has landed (two younger ones may be in flight), and
+        // after the barrier everybody's; the buffer of stage st - 1 is free for stage st + 3
+        __builtin_amdgcn_s_waitcnt(I4L_VMCNT(kPairStages - 2));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        issue(st + kPairStages - 1);
+        const uint8_t *stage = lds + (st % kPairStages) * kTinyStageBytes;
+        const v4i px = *(const v4i *)(stage + x_rd);
+        const v4i pw = *(const v4i *)(stage + w_rd);
+        if (st > 0) {  // stage st - 1, behind the reads of stage st
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(xlo, wlo, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(xhi, whi, acc, 0, 0, 0);
+        }
+        xlo = (px << 4) & himask;
+        xhi = px & himask;
+        wlo = (pw << 4) & himask;
+        whi = pw & himask;
+    }
+    acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(xlo, wlo, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(xhi, whi, acc, 0, 0, 0);
+
+    // ---- the upper group's sums go through LDS to the lower group, which stores the tile
+    __builtin_amdgcn_s_waitcnt(I4L_VMCNT(0));  // the loads past the end have landed too
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int *merge = (int *)lds + (size_t)quad * 16 * 64 + lane;
+    if (half == 1) {
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            merge[t * 64] = acc[t];
+    }
+    __syncthreads();
+    if (half == 1)
+        return;
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+        acc[t] = (acc[t] + merge[t * 64]) >> 8;  // both operands carried a factor 16
+    // accumulator t is  m = 8 (t / 4) + 4 (lane / 32) + t % 4,  n = lane % 32  of the quadrant
+    const int mw = m0 + wm * kFrag + 4 * (lane >> 5);
+    const int nw = n0 + wn * kFrag + (lane & 31);
+    int32_t *out = Y + (size_t)mw * N + nw;
+    // a half-width output as a whole (launch_mfma sends at most a few hundred tiles here)
+    __amdgpu_buffer_rsrc_t rsrc16 = __builtin_amdgcn_make_buffer_rsrc(Y, 0, (int)((unsigned)M * (unsigned)N * 2u), 0x00020000);
+    if (!HALF_OUT && !ep.bias && !ep.row_scale && !ep.col_scale && !ep.out) {
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const int dm = 8 * (t / 4) + (t % 4);
+            if (mw + dm < M && nw < N)
+                out[(size_t)dm * N] = acc[t];
+        }
+        return;
+    }
+    const int nn = min(nw, N - 1);
+    const int bias_v = ep.bias ? ep.bias[nn] : 0;
+    const float cs_v = ep.col_scale ? ep.col_scale[nn] : 1.f;
+    float rs[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+        rs[t] = ep.row_scale ? ep.row_scale[min(mw + 8 * (t / 4) + (t % 4), M - 1)] : 1.f;
+    if constexpr (!HALF_OUT) {
+        int v[16];  // the values first (opaque: they stay here), then the stores, each behind nothing but its bounds test
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            v[t] = opaque(epilogue_value32(ep, acc[t], bias_v, rs[t], cs_v));
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const int dm = 8 * (t / 4) + (t % 4);
+            if (mw + dm < M && nw < N)
+                out[(size_t)dm * N] = v[t];
+        }
+    } else {
+        // (stores through a descriptor over the whole output, as in mfma_pair_kernel)
+        const unsigned col_off = nw < N ? (unsigned)nw * 2u : 0x40000000u;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const int dm = 8 * (t / 4) + (t % 4);
+            const unsigned row_off = mw + dm < M ? (unsigned)(mw + dm) * (unsigned)N * 2u : 0x80000000u;
+            __builtin_amdgcn_raw_buffer_store_b16((unsigned short)epilogue_value16(ep, acc[t], bias_v, rs[t], cs_v),
+                                                  rsrc16, row_off + col_off, 0, 0);
+        }
+    }
+}
+
 // 256 x 256 tile, eight wavefronts of 128 (m) x 64 (n), one workgroup per CU, two
 // wavefronts per SIMD: the large-shape configuration.
 using CfgLarge = TileConfig<2, 4, 4, 2, 4, 1>;
@@ -1092,8 +1235,17 @@ hipError_t launch_mfma(const void *a, const void *b, void *c, int m, int n, int 
     // Few 128 x 128 tiles per CU: the form whose two waves per SIMD split K.
     const int pair_m = (m + kPairTile - 1) / kPairTile, pair_n = (n + kPairTile - 1) / kPairTile;
     // ... and so few that smaller tiles leave the busiest CU less to do (kernels_grid.hip).
-    if (grid_preferred(m, n, dev))
+    if (grid_preferred(m, n, k, dev))
         return launch_grid(a, b, c, m, n, k, ep, dev, stream);
+    // ... with K too short for that form: 64 x 64 tiles where 128 x 128 ones would leave half of the CUs
+    // idle or more (1024 x 1024 x 640 6.9 -> 4.6 us).
+    if ((long)pair_m * pair_n * 2 <= dev.cu_count) {
+        const int tiny_m = (m + kTinyTile - 1) / kTinyTile, tiny_n = (n + kTinyTile - 1) / kTinyTile;
+        auto *kern = ep.out >= kOutF16 ? mfma_pair64_kernel<true> : mfma_pair64_kernel<false>;
+        kern<<<(unsigned)(tiny_m * tiny_n), 512, kTinyLdsBytes, stream>>>((const uint8_t *)a, (const uint8_t *)b, (int32_t *)c, m, n, k,
+                                                                          tiny_m, tiny_n, ep);
+        return hipGetLastError();
+    }
     if ((long)pair_m * pair_n <= (long)dev.cu_count * kPairRounds) {
         const bool deep = (long)pair_m * pair_n <= dev.cu_count, half_out = ep.out >= kOutF16;
         auto *kern = deep ? (half_out ? mfma_pair_kernel<true, true> : mfma_pair_kernel<true, false>)

@@ -470,16 +470,22 @@ def test_small_grid_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     (70, 33, 128, False), (96, 96, 256, False), (65, 300, 896, False), (129, 511, 2048, False),
     # 64 x 32 tiles, four waves and (K > 2048) eight
     (257, 1000, 384, False), (640, 600, 1920, False), (257, 1000, 2176, False), (639, 601, 2432, False),
-    # 64 x 64 tiles
-    (515, 2050, 128, False), (1025, 1000, 640, False), (1000, 1111, 1152, False),
-    # 64 x 96 tiles
-    (1030, 1930, 128, False), (2049, 1100, 1152, False), (1000, 3000, 896, False),
+    # 64 x 64 tiles: K of whole stages, of 1408 and more with three, one and two pieces in the last one
+    (515, 2050, 1024, False), (1025, 1000, 1408, False), (515, 2050, 1664, False), (1000, 1111, 1792, False),
+    # 64 x 96 tiles, up to 128 tiles of 128 x 128 and beyond (K of whole stages, 2816 and more, 3328 and more)
+    (1030, 1930, 1024, False), (1100, 1000, 1920, False), (2049, 1100, 1536, False), (1000, 3000, 2816, False), (1000, 3000, 3328, False),
+    # ... beyond, because 128 x 128 tiles would pad a quarter more
+    (130, 8500, 128, False), (130, 8500, 640, False),
+    # shorter K on the form whose waves split every stage in two, with 64 x 64 and with 128 x 128 tiles
+    (515, 2050, 128, False), (1025, 1000, 640, False), (1000, 1111, 1152, False), (1025, 1000, 1280, False),
+    (1030, 1930, 128, False), (2049, 1100, 1152, False), (1000, 3000, 896, False), (1000, 3000, 3200, False),
     # each of them split over K across workgroups, with odd numbers of pieces per slice
     (65, 200, 8448, True), (200, 700, 8960, True), (250, 2300, 12544, True), (66, 60, 8320, True)])
 def test_tiles_of_the_small_grid_form(gpu, host_threads, m, n, k, split):
-    """Every tile of the small-grid form at its edges: rows and columns past the tile, K that
-    ends inside a stage, fewer stages than the ring holds, all output types; the split over K
-    called several times (its counters go back to zero) and without a workspace."""
+    """Every tile of the small-grid form at its edges, and the forms that take shorter K: rows and
+    columns past the tile, K that ends inside a stage, fewer stages than the ring holds, all output
+    types; the split over K called several times (its counters go back to zero) and without a
+    workspace."""
     import torch
 
     import int4linear_amd as lib
