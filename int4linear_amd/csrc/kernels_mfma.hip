@@ -1163,11 +1163,13 @@ hipError_t launch_mfma_tile(const void *a, const void *b, void *c, int m, int n,
     return hipErrorInvalidValue;
 }
 
-// K-slices per 128 x 128 tile of mfma_pair_kernel, for shapes with more tiles than the small-grid
-// form splits and long K: at most half as many tiles as CUs at K >= 12288 (512 x 4096 x 14336
-// 35.6 us split, 52 us as one tile per workgroup): the largest divisor of the stage count that
-// keeps at least eight stages per slice, at most eight slices, and at most half a work item
-// per slot.
+// K-slices per 128 x 128 tile of mfma_pair_kernel, for long K and more tiles than the small-grid
+// form splits, or as many whose stages its few slices do not divide: at most half as many tiles as
+// CUs at K >= 12288 (512 x 4096 x 14336 35.6 us split, 52 us as one tile per workgroup): the
+// largest divisor of the stage count that keeps at least eight stages per slice, at most eight
+// slices, and at most half a work item per slot.  Up to a quarter as many tiles as CUs the unsplit
+// small-grid form is as fast as two or three slices (512 x 2048 x 12672 21.4, 22.4 us in three), not as
+// more (300 x 2000 x 16000 25.0, 21.0 in five).
 int mfma_ksplit(int m, int n, int k, const DeviceInfo &dev)
 {
     if (!mfma_supports(m, n, k))
@@ -1175,7 +1177,7 @@ int mfma_ksplit(int m, int n, int k, const DeviceInfo &dev)
     const long tiles = (long)((m + CfgMedium::BM - 1) / CfgMedium::BM) * ((n + CfgMedium::BN - 1) / CfgMedium::BN);
     const long slots = (long)dev.cu_count * CfgMedium::OCC;
     const int stages = k / kStageK;
-    if (tiles * 2 > dev.cu_count || tiles * 4 <= dev.cu_count || stages < 96)
+    if (tiles * 2 > dev.cu_count || tiles * 16 <= dev.cu_count || stages < 96)
         return 1;
     long limit = slots / (2 * tiles);
     if (limit > 8)
@@ -1184,7 +1186,7 @@ int mfma_ksplit(int m, int n, int k, const DeviceInfo &dev)
     for (int d = 2; d <= limit; ++d)
         if (stages % d == 0 && stages / d >= 8)
             best = d;
-    return best;
+    return tiles * 4 <= dev.cu_count && best < 4 ? 1 : best;
 }
 
 // The small-grid form's split: few tiles at K >= 8192, more of them at K >= 12288.

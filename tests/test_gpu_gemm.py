@@ -735,10 +735,12 @@ def test_split_k_form_of_the_fp6_kernel(gpu, host_threads, m, n, k):
 
 
 @pytest.mark.parametrize("m, n, k", [(128, 4096, 14336), (300, 520, 12288), (1024, 512, 14336), (100, 300, 8192),
-                                     (140, 1000, 12288), (200, 136, 16384)])
+                                     (140, 1000, 12288), (200, 136, 16384),
+                                     (512, 4096, 12288), (500, 3998, 12544), (300, 1999, 16000)])
 def test_split_k_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
-    """Few tiles and long K: automatic dispatch splits K over workgroups (partial sums in the
-    internal workspace, a second kernel adds them and applies the epilogue)."""
+    """Few tiles and long K: automatic dispatch splits K over workgroups, with partial sums in the
+    internal workspace: of the small-grid form's tiles, which meet inside the launch, or (the last three
+    shapes) of 128 x 128 tiles, whose slabs a second kernel adds up before it applies the epilogue."""
     import torch
 
     import int4linear_amd as lib
@@ -751,7 +753,6 @@ def test_split_k_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     lib.init()
     assert lib.workspace_bytes(m, n, k) > 0 and lib.workspace_bytes(m, n, k) % (m * n * 4) == 0
     assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="auto"), want)
-    # the epilogue moves into the second kernel
     rng = np.random.default_rng(m + k)
     bias = rng.integers(-1000, 1000, size=n, dtype=np.int32)
     rs = rng.uniform(0.1, 2.0, size=m).astype(np.float32)
