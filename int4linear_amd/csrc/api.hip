@@ -140,7 +140,7 @@ bool fp6_worthwhile(int m, int n, int k, const DeviceInfo &dev, size_t limit)
 {
     const long tiles = (long)((m + 255) / 256) * ((n + 255) / 256);
     const bool pays = (tiles >= 128 && k >= 8192) || (tiles >= 144 && k >= 3072) || (tiles >= 384 && k >= 1024);
-    return pays && fp6_supports(m, n, k) && fp6_workspace_bytes(m, n, k, dev) <= limit;
+    return pays && fp6_supports(m, n, k) && fp6_workspace_bytes(m, n, k, dev, limit) <= limit;
 }
 
 // K that is not a multiple of 128 fits neither the int8 nor the weight-streaming kernel,
@@ -149,7 +149,7 @@ bool fp6_worthwhile(int m, int n, int k, const DeviceInfo &dev, size_t limit)
 bool fp6_for_ragged_k(int m, int n, int k, const DeviceInfo &dev, size_t limit)
 {
     return (k % 128) != 0 && fp6_supports(m, n, k) && (double)m * n * k >= (double)(1 << 22) &&
-           fp6_workspace_bytes(m, n, k, dev) <= limit;
+           fp6_workspace_bytes(m, n, k, dev, limit) <= limit;
 }
 
 // The current device's record, set up if it has not been yet; without a usable device an
@@ -241,12 +241,13 @@ int acquire_workspace(PerDevice *pd, size_t need, hipStream_t stream, void **out
 int run_fp6(PerDevice *pd, const void *a, const void *b, void *c, int m, int n, int k,
             const Epilogue &ep, Workspace source, bool capturing, hipStream_t stream)
 {
-    const size_t need = fp6_workspace_bytes(m, n, k, pd->info);
+    const size_t limit = source == Workspace::Static ? kStaticScratchBytes : g_workspace_limit.load();
+    const size_t need = fp6_workspace_bytes(m, n, k, pd->info, limit);
     hipError_t e;
     if (source == Workspace::Static) {
         if (need > kStaticScratchBytes)
             return INT4LINEAR_ERR_SCRATCH;
-        e = launch_fp6(a, b, c, m, n, k, pd->scratch, pd->arrivals + kSkinnyArrivalWords, ep, pd->info, stream);
+        e = launch_fp6(a, b, c, m, n, k, pd->scratch, need, pd->arrivals + kSkinnyArrivalWords, ep, pd->info, stream);
     } else {
         if (source == Workspace::None || capturing)
             return INT4LINEAR_ERR_UNSUPPORTED;
@@ -255,7 +256,7 @@ int run_fp6(PerDevice *pd, const void *a, const void *b, void *c, int m, int n, 
         const int st = acquire_workspace(pd, need, stream, &ws);
         if (st != INT4LINEAR_OK)
             return st;
-        e = launch_fp6(a, b, c, m, n, k, ws, pd->arrivals, ep, pd->info, stream);
+        e = launch_fp6(a, b, c, m, n, k, ws, need, pd->arrivals, ep, pd->info, stream);
     }
     return e == hipSuccess ? INT4LINEAR_OK : fail_hip(e);
 }
@@ -661,7 +662,7 @@ size_t int4linear_workspace_bytes(int m, int n, int k)
     const DeviceInfo info = current_device_info();
     const int kernel = pick_kernel(m, n, k, info, g_workspace_limit.load());
     if (kernel == INT4LINEAR_KERNEL_FP6)
-        return fp6_workspace_bytes(m, n, k, info);
+        return fp6_workspace_bytes(m, n, k, info, g_workspace_limit.load());
     if (kernel == INT4LINEAR_KERNEL_MFMA || kernel == INT4LINEAR_KERNEL_SKINNY) {
         // the split-K forms need the device's CU count: unknown only without a device
         if (info.cu_count == 0)
@@ -716,7 +717,7 @@ int version_kernel(int version, int m, int n, int k, const DeviceInfo &info)
     case 21:
         return INT4LINEAR_KERNEL_AUTO;
     case 20:
-        if (fp6_supports(m, n, k) && fp6_workspace_bytes(m, n, k, info) <= g_workspace_limit.load() &&
+        if (fp6_supports(m, n, k) && fp6_workspace_bytes(m, n, k, info, g_workspace_limit.load()) <= g_workspace_limit.load() &&
             !skinny_preferred(m, n, k, info))
             return INT4LINEAR_KERNEL_FP6;
         [[fallthrough]];

@@ -174,9 +174,10 @@ hipError_t launch_mfma_tile(const void *a, const void *b, void *c, int m, int n,
 // (256-byte aligned), then runs the GEMM on it.  Requires K % 8 == 0, K < 2^18.  With few
 // output tiles and long K the GEMM is split over K (it depends on the device's CU count and is
 // not while that is unknown): partial sums in the same workspace, arrivals counted at
-// `arrivals` as by launch_skinny_ksplit below.
+// `arrivals` as by launch_skinny_ksplit below.  `limit`: the most the workspace may be; a split whose
+// partial sums alone would exceed it is left out where the unsplit form takes the shape as well.
 bool fp6_supports(int m, int n, int k);
-size_t fp6_workspace_bytes(int m, int n, int k, const DeviceInfo &dev);
+size_t fp6_workspace_bytes(int m, int n, int k, const DeviceInfo &dev, size_t limit);
 hipError_t fp6_init(const DeviceInfo &dev);
 // The two halves of launch_fp6 on caller-owned buffers: an operand of `rows` rows converts
 // into fp6_operand_bytes(rows, k) bytes (256-byte aligned); the GEMM runs on two of those.
@@ -184,9 +185,10 @@ size_t fp6_operand_bytes(int rows, int k);
 hipError_t launch_fp6_convert(const void *src, void *dst, int rows, int k, hipStream_t stream);
 hipError_t launch_fp6_gemm(const void *a_conv, const void *b_conv, void *c, int m, int n, int k,
                            const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
-hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
-                      const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
-// Its GEMM for grids of few tiles (kernels_fp6_grid.hip): fp6_grid_slices() slices of K across
+hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, size_t workspace_bytes,
+                      unsigned *arrivals, const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream);
+// Its GEMM for grids of few tiles (kernels_fp6_grid.hip; fp6_grid_preferred: where it may be the faster
+// one, with regard to the grid alone): fp6_grid_slices() slices of K across
 // workgroups with `bytes` bytes of partial sums (1 and 0: not split).
 hipError_t fp6_grid_init(const DeviceInfo &dev);
 bool fp6_grid_preferred(int m, int n, const DeviceInfo &dev);

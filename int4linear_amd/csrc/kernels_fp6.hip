@@ -24,12 +24,14 @@
 //     the workspace is already in the order lanes consume it, global->LDS is a linear
 //     direct-to-LDS copy, LDS->VGPR is one 16-byte and one 8-byte read per lane per
 //     fragment at consecutive addresses (no swizzle, no bank conflicts), and the main loop
-//     contains no VALU work at all.  (Grids of few tiles run on kernels_fp6_grid.hip.)
+//     contains no VALU work at all.  Grids of few tiles run on kernels_fp6_grid.hip, or here as
+//     slices of K whose partial sums a second kernel adds up (plan_gemm).
 //
 // Order of k inside a fragment is whatever the converter produces; it only has to be the
 // same for both operands, which it is because both go through the same converter.
 #include "kernels.h"
 #include "fp6_format.h"
+#include "grid_tail.h"
 
 #include <type_traits>
 #include <utility>
@@ -266,7 +268,11 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::WAVES_N;
     const int wn = wave % C::WAVES_N;
-    const int KT = K / kStageK;
+    // gridDim.y > 1: few tiles and long K.  Slice y covers KT of the KT_all stages and stores its plain
+    // partial sums into slab y of Y (M * N int32 each), which a second kernel adds up.
+    const int KT_all = K / kStageK;
+    const int KT = KT_all / (int)gridDim.y;
+    const int slice = blockIdx.y;
     const int total_tiles = tiles_m * tiles_n;
     const int nblk = gridDim.x;
     const int bid = blockIdx.x;
@@ -293,8 +299,8 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
         tile_coords(bid + it * nblk, total_tiles, tiles_m, tiles_n, tm, tn);
         if constexpr (!Parts::kOwnTile)
             tm = tn = 0;
-        xptr = XW + (size_t)tm * KT * kOperandStageBytes;
-        wptr = WW + (size_t)tn * KT * kOperandStageBytes;
+        xptr = XW + ((size_t)tm * KT_all + (size_t)slice * KT) * kOperandStageBytes;
+        wptr = WW + ((size_t)tn * KT_all + (size_t)slice * KT) * kOperandStageBytes;
     };
     auto ld_chunk = [&](auto c, unsigned ring) {  // c < CH/2: X half, else W half; ring: the buffer's offset
         constexpr int cc = decltype(c)::value;
@@ -508,7 +514,7 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
             const int m0 = tm * kTileRows, n0 = tn * kTileRows;
             const int rows_left = M - m0;  // > 0
             const int cols_left = N - n0;  // > 0
-            int32_t *ybase = Y + (size_t)m0 * N + n0;
+            int32_t *ybase = Y + (size_t)slice * (size_t)M * (size_t)N + (size_t)m0 * N + n0;
             const size_t slab_rows = rows_left < kTileRows ? rows_left : kTileRows;
             const size_t extent = ((slab_rows - 1) * (size_t)N + (size_t)(cols_left < kTileRows ? cols_left : kTileRows)) * 4u;
             __amdgpu_buffer_rsrc_t rsrc =
@@ -576,7 +582,7 @@ __global__ __launch_bounds__(C::THREADS, C::OCC) void fp6_gemm_kernel(
                     }
                 } else {
                     // The half-width kinds: a descriptor over the same tile of an output of
-                    // two-byte elements, every offset halved.
+                    // two-byte elements, every offset halved (slices of K are int32 always).
                     __amdgpu_buffer_rsrc_t rsrc16 = __builtin_amdgcn_make_buffer_rsrc(
                         (uint8_t *)Y + ((size_t)m0 * N + n0) * 2u, 0, (int)(extent / 2u), 0x00020000);
 #pragma unroll
@@ -643,14 +649,71 @@ bool fp6_supports(int m, int n, int k)
     return m >= 1 && n >= 1 && m <= kMaxRows && n <= kMaxRows && k >= 8 && k % 8 == 0 && k <= (1 << 18) - kStageK;
 }
 
-size_t fp6_workspace_bytes(int m, int n, int k, const DeviceInfo &dev)
+namespace {
+
+// How a GEMM of converted operands runs.
+struct GemmPlan {
+    bool grid = false;   // on kernels_fp6_grid.hip
+    int slices = 1;      // of K
+    size_t partial = 0;  // bytes of their partial sums
+};
+
+// The most slices of K of the large kernel that leave a workgroup per CU, 2048 k per slice and equal slices.
+int large_slices(long tiles, int stages, const DeviceInfo &dev)
 {
+    if (tiles * 4 > dev.cu_count)  // (two slices of 128 tiles gain nothing over 128 unsplit ones)
+        return 1;
+    for (int d = kGridMaxSlices; d > 1; --d)
+        if (tiles * d <= dev.cu_count && stages % d == 0 && stages / d >= 16)
+            return d;
+    return 1;
+}
+
+// `room`: the most bytes the large kernel's partial sums may take.  Grids of up to one 64 x 64 tile per CU run on those
+// tiles.  Beyond, they read every operand four times as often as 256 x 256 tiles do, and what the larger
+// ones lose is idle CUs, or the partial sums' way to memory and back: the least of the three
+// estimates below, in us, without the converter.  us, 64 x 64 / 256 x 256 in slices of K (their number) / unsplit:
+// 1024 x 4096 x 8192 54 / 65 (4) / -; x 12296 74 / - / 70; x 16384 98 / 85 (4) / -; x 20488 115 / - / 109; x
+// 28672 161 / 116 (4) / -; 768 x 3072 x 16376 72 / 55 (4) / -; 1000 x 3000 x 12296 58 / - / 67; 512 x 4096 x 16384
+// 60 / 73 (8) / -, x 28680 98 / 80 (5) / -; 600 x 3300 x 28680 121 / 89 (5) / -.  Unsplit 256 x 256 tiles fall behind
+// again once the operands outgrow the memory-side cache (512 x 8192 x 24584, 160 MB: 158 / - / 161; x 32776 252 / - / 281).
+GemmPlan plan_gemm(int m, int n, int k, const DeviceInfo &dev, size_t room)
+{
+    constexpr size_t kCachedOperands = 140u << 20;
+    const long tiles64 = grid_tiles(m, n, 64, 64), tiles = grid_tiles(m, n, kTileRows, kTileRows);
+    const int stages = (k + kStageK - 1) / kStageK;
+    GemmPlan p;
+    p.grid = fp6_grid_preferred(m, n, dev);
+    if (!p.grid)
+        return p;
+    if (tiles64 > dev.cu_count) {
+        const double per_k = 3.7e-3 * k;
+        const double small = 8 + 0.98e-3 * k * (double)((tiles64 + dev.cu_count - 1) / dev.cu_count);
+        const bool cached = operand_ws_bytes(m, k) + operand_ws_bytes(n, k) <= kCachedOperands;
+        const double whole = cached ? 10 + per_k : small;
+        const int d = large_slices(tiles, stages, dev);
+        const size_t slabs = (size_t)d * (size_t)m * (size_t)n * 4u;
+        const double split = d > 1 && slabs <= room ? 10 + per_k / d + (2 * d + 1) * 4. * m * n / 4.5e6 : small;
+        if (split < small && split <= whole)
+            return GemmPlan{false, d, slabs};
+        if (whole < small)
+            return GemmPlan{};
+    }
+    p.slices = fp6_grid_slices(m, n, k, dev, &p.partial);
+    return p;
+}
+
+}  // namespace
+
+size_t fp6_workspace_bytes(int m, int n, int k, const DeviceInfo &dev, size_t limit)
+{
+    const size_t operands = operand_ws_bytes(m, k) + operand_ws_bytes(n, k);
+    if (dev.cu_count <= 0)
+        return operands;
     // (partial sums: whole multiples of the output's size)
     const size_t out = (size_t)m * (size_t)n * 4u;
-    size_t partial = 0;
-    if (dev.cu_count > 0)
-        fp6_grid_slices(m, n, k, dev, &partial);
-    return operand_ws_bytes(m, k) + operand_ws_bytes(n, k) + (partial + out - 1) / out * out;
+    const size_t partial = plan_gemm(m, n, k, dev, limit > operands ? limit - operands : 0).partial;
+    return operands + (partial + out - 1) / out * out;
 }
 
 hipError_t fp6_init(const DeviceInfo &dev)
@@ -707,21 +770,22 @@ hipError_t launch_fp6_convert(const void *src, void *dst, int rows, int k, hipSt
 
 namespace {
 
-hipError_t launch_tiles(const void *a_conv, const void *b_conv, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
-                        hipStream_t stream)
+// slices > 1: `c` is as many slabs of m * n partial sums and `ep` must be empty.
+hipError_t launch_tiles(const void *a_conv, const void *b_conv, void *c, int m, int n, int k, int slices, const Epilogue &ep,
+                        const DeviceInfo &dev, hipStream_t stream)
 {
     using C = Fp6Cfg;
     const int tiles_m = (m + kTileRows - 1) / kTileRows;
     const int tiles_n = (n + kTileRows - 1) / kTileRows;
     const long total = (long)tiles_m * tiles_n;
-    if (total > 0x7fffffffL || (size_t)kTileRows * (size_t)n * 4u > 0x40000000ull)
+    if (total > 0x7fffffffL || (size_t)kTileRows * (size_t)n * 4u > 0x40000000ull || (slices > 1 && ep.out >= kOutF16))
         return hipErrorInvalidValue;
     long grid = (long)dev.cu_count * C::OCC;
     if (grid > total)
         grid = total;
     auto *kern = ep.out >= kOutF16 ? fp6_gemm_kernel<C, true> : fp6_gemm_kernel<C>;
-    kern<<<(unsigned)grid, C::THREADS, kLdsBytes, stream>>>((const uint8_t *)a_conv, (const uint8_t *)b_conv, (int32_t *)c, m, n,
-                                                             padded_k(k), tiles_m, tiles_n, ep);
+    kern<<<dim3((unsigned)grid, (unsigned)slices), C::THREADS, kLdsBytes, stream>>>(
+        (const uint8_t *)a_conv, (const uint8_t *)b_conv, (int32_t *)c, m, n, padded_k(k), tiles_m, tiles_n, ep);
     return hipGetLastError();
 }
 
@@ -730,26 +794,27 @@ hipError_t launch_tiles(const void *a_conv, const void *b_conv, void *c, int m, 
 hipError_t launch_fp6_gemm(const void *a_conv, const void *b_conv, void *c, int m, int n, int k,
                            const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
 {
-    if (fp6_grid_preferred(m, n, dev))
+    if (plan_gemm(m, n, k, dev, 0).grid)
         return launch_fp6_grid(a_conv, b_conv, c, m, n, k, 1, nullptr, nullptr, ep, dev, stream);
-    return launch_tiles(a_conv, b_conv, c, m, n, k, ep, dev, stream);
+    return launch_tiles(a_conv, b_conv, c, m, n, k, 1, ep, dev, stream);
 }
 
-hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, unsigned *arrivals,
-                      const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
+hipError_t launch_fp6(const void *a, const void *b, void *c, int m, int n, int k, void *workspace, size_t workspace_bytes,
+                      unsigned *arrivals, const Epilogue &ep, const DeviceInfo &dev, hipStream_t stream)
 {
     uint8_t *xws = (uint8_t *)workspace;
     uint8_t *wws = xws + operand_ws_bytes(m, k);
-    const bool grid = fp6_grid_preferred(m, n, dev);
-    hipError_t e = launch_convert_jobs(make_job(a, xws, m, !grid), make_job(b, wws, n, !grid), k, stream);
+    uint8_t *partial = wws + operand_ws_bytes(n, k);
+    const GemmPlan p = plan_gemm(m, n, k, dev, workspace_bytes - (size_t)(partial - xws));
+    hipError_t e = launch_convert_jobs(make_job(a, xws, m, !p.grid), make_job(b, wws, n, !p.grid), k, stream);
     if (e != hipSuccess)
         return e;
-    if (!grid)
-        return launch_tiles(xws, wws, c, m, n, k, ep, dev, stream);
-    // Few tiles and long K: slices of K across workgroups, partial sums behind the operands.
-    size_t partial = 0;
-    const int slices = fp6_grid_slices(m, n, k, dev, &partial);
-    return launch_fp6_grid(xws, wws, c, m, n, k, slices, wws + operand_ws_bytes(n, k), arrivals, ep, dev, stream);
+    if (p.grid)
+        return launch_fp6_grid(xws, wws, c, m, n, k, p.slices, partial, arrivals, ep, dev, stream);
+    if (p.slices == 1)
+        return launch_tiles(xws, wws, c, m, n, k, 1, ep, dev, stream);
+    e = launch_tiles(xws, wws, partial, m, n, k, p.slices, Epilogue{}, dev, stream);
+    return e == hipSuccess ? launch_splitk_reduce(partial, c, (size_t)m * (size_t)n, p.slices, n, ep, stream) : e;
 }
 
 }  // namespace int4linear

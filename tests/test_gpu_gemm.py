@@ -700,11 +700,12 @@ def test_few_rows_against_any_k(gpu, host_threads, m, n, k):
 
 
 @pytest.mark.parametrize("m, n, k", [(300, 2049, 8192), (257, 1000, 4096), (512, 1024, 14336), (300, 520, 16392),
-                                     (1024, 4096, 14336)])
+                                     (1024, 4096, 14336), (600, 3301, 16376)])
 def test_split_k_form_of_the_fp6_kernel(gpu, host_threads, m, n, k):
-    """64 tiles of 256 x 256 or fewer and long K: the FP6 GEMM runs K-slices of every tile on
-    their own CUs (partial sums in slabs behind the converted operands in the internal
-    workspace), a second kernel adds them up and applies the epilogue."""
+    """64 tiles of 256 x 256 or fewer and long K: the FP6 GEMM runs slices of K on CUs of their own,
+    with partial sums behind the converted operands in the internal workspace: of 64 x 64 and smaller
+    tiles, which meet inside the launch, or (the last two shapes) of 256 x 256 tiles, whose slabs a
+    second kernel adds up before it applies the epilogue."""
     import torch
 
     import int4linear_amd as lib
@@ -773,6 +774,57 @@ def test_split_k_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
         assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="auto"), want)
     finally:
         lib.set_workspace_limit(1 << 30)
+
+
+def test_fp6_forms_and_their_workspace(gpu, host_threads):
+    """Few tiles: 64 x 64 ones need room for the operands alone; 256 x 256 ones in slices of K, for a slab
+    of partial sums per slice on top, and where a limit leaves no room for the slabs the call runs
+    without them."""
+    import torch
+
+    import int4linear_amd as lib
+
+    lib.init()
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes below are those of 256 compute units")
+    operands = lambda m, n, k: lib.fp6_operand_bytes(m, k) + lib.fp6_operand_bytes(n, k)
+    for (m, n, k), slices in (((1024, 4096, 16376), 4), ((600, 3301, 16376), 4), ((512, 4096, 28680), 5), ((1536, 2560, 28680), 3),
+                              ((1024, 4096, 12296), 0), ((512, 4096, 16376), 0), ((1000, 3000, 4104), 0)):
+        assert lib.workspace_bytes(m, n, k) == operands(m, n, k) + slices * m * n * 4, (m, n, k)
+    m, n, k = 600, 3301, 16376
+    x, w = helpers.uniform_s4(3800, m, k), helpers.uniform_s4(3801, n, k)
+    want = oracle.linear_ref(x, w, threads=host_threads)
+    xp, wp = helpers.pack_bytes(x), helpers.pack_bytes(w)
+    lib.set_workspace_limit(operands(m, n, k) + m * n * 4)
+    try:
+        assert lib.kernel_for_shape(m, n, k) == "fp6" and lib.workspace_bytes(m, n, k) == operands(m, n, k)
+        assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="auto"), want)
+    finally:
+        lib.set_workspace_limit(1 << 30)
+    assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="auto"), want)
+
+
+@pytest.mark.parametrize("m, n, k", [(1024, 4096, 12296), (2000, 2048, 16384)])
+def test_whole_fp6_tiles_where_small_ones_are_many(gpu, host_threads, m, n, k):
+    """Four 64 x 64 tiles per CU and long K on 256 x 256 tiles unsplit: through the workspace and on
+    caller-owned operands."""
+    import torch
+
+    import int4linear_amd as lib
+
+    x, w = helpers.uniform_s4(3900 + m, m, k), helpers.uniform_s4(3901 + n, n, k)
+    rows = np.linspace(0, m - 1, 48, dtype=int)
+    want = oracle.linear_ref(x[rows], w, threads=host_threads)
+    xp, wp = helpers.pack_bytes(x), helpers.pack_bytes(w)
+    assert np.array_equal(helpers.run_gemm(xp, wp, m, n, k, kernel="fp6")[rows], want)
+    xd, wd = helpers.to_device_bytes(xp), helpers.to_device_bytes(wp)
+    xc = torch.empty(lib.fp6_operand_bytes(m, k), dtype=torch.uint8, device="cuda:0")
+    wc = torch.empty(lib.fp6_operand_bytes(n, k), dtype=torch.uint8, device="cuda:0")
+    lib.fp6_convert(xd, xc, m, k)
+    lib.fp6_convert(wd, wc, n, k)
+    y = torch.full((m, n), -1, dtype=torch.int32, device="cuda:0")
+    lib.gemm_fp6_converted(xc, wc, y, m, n, k)
+    assert np.array_equal(y.cpu().numpy()[rows], want)
 
 
 def test_concurrent_host_threads(gpu, host_threads):
