@@ -29,12 +29,13 @@ def _ptr(obj) -> int:
 def _current_stream() -> int:
     """The handle torch.cuda.current_stream().cuda_stream gives, asked for without the Stream object that
     call makes: 2.7 us, longer than the smallest kernels run and more than a third of a call's 7.4 us on
-    the host, against 0.3."""
+    the host, against 0.3.  (A torch without that private function is asked the long way.)"""
     import torch
 
-    if not torch.cuda.is_initialized():  # (torch sets itself up, or says why it cannot)
+    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw_stream is None or not torch.cuda.is_initialized():  # (torch sets itself up, or says why it cannot)
         return torch.cuda.current_stream().cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return raw_stream(torch.cuda.current_device())
 
 
 def init() -> None:

@@ -153,3 +153,18 @@ def test_bench_refuses_more_than_one_gpu():
     root = Path(__file__).resolve().parent.parent
     r = subprocess.run([sys.executable, str(root / "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode == 2 and "one GPU" in r.stderr and r.stdout.strip() == ""
+
+
+def test_stream_of_a_call_without_torchs_private_function(monkeypatch):
+    """torch._C._cuda_getCurrentRawStream is not part of torch's interface: without it the stream's
+    handle comes from torch.cuda.current_stream()."""
+    import types
+
+    import torch
+
+    from int4linear_amd import api
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=1234))
+    assert api._current_stream() == 1234
