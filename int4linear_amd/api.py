@@ -32,10 +32,12 @@ def _current_stream() -> int:
     the host, against 0.3.  (A torch without that private function is asked the long way.)"""
     import torch
 
-    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw_stream is None or not torch.cuda.is_initialized():  # (torch sets itself up, or says why it cannot)
-        return torch.cuda.current_stream().cuda_stream
-    return raw_stream(torch.cuda.current_device())
+    if torch.cuda.is_initialized():  # (else torch sets itself up, or says why it cannot)
+        try:
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        except AttributeError:
+            pass
+    return torch.cuda.current_stream().cuda_stream
 
 
 def init() -> None:
