@@ -439,17 +439,20 @@ hipError_t grid_init(const DeviceInfo &)
     return e;
 }
 
-// 64 x 32 and 32 x 32 tiles always.  The larger ones once K is long enough: up to 128 tiles of 128 x 128
-// mfma_pair64_kernel is the other choice, beyond mfma_pair_kernel, whose tiles must not pad a quarter
-// more for K to decide (130 x 8500, 134 tiles against 267: 1024 8.8 / 6.6 us with bf16 output).
+// Up to 128 tiles of 128 x 128, where mfma_pair64_kernel is the other choice: 64 x 32 and 32 x 32 tiles
+// always, the larger ones once K is long enough.  Beyond, where it is mfma_pair_kernel: always up to
+// 64 rows, half of what its tiles hold, and where 64 x 64 tiles fit the device two to a CU (int32, us, that
+// kernel / this one: 700 x 2712, 473 of them, x 256 6.8 / 6.0, x 1152 8.9 / 7.7; 257 x 5464, 430, x 1920 10.5 / 8.2), so
+// that they are the ones chosen; with 64 x 96 tiles once K is long enough (580 x 3500 x 640 7.5 / 8.5).
 bool grid_preferred(int m, int n, int k, const DeviceInfo &dev)
 {
     if (few_tiles(m, n, dev)) {
         const Tile tile = choose_tile(m, n, k, dev);
         return (tile != Tile::k64x64 && tile != Tile::k64x96) || long_enough(k, 1408);
     }
-    const long tiles = grid_tiles(m, n, 64, 96);
-    return tiles <= 2l * dev.cu_count && (tiles * (64 * 96) * 5 <= grid_tiles(m, n, 128, 128) * (128 * 128) * 4 || long_enough(k, k % 512 == 128 ? 3328 : 2816));
+    if (grid_tiles(m, n, 64, 96) > 2l * dev.cu_count)
+        return false;
+    return m <= 64 || grid_tiles(m, n, 64, 64) <= 2l * dev.cu_count || long_enough(k, k % 512 == 128 ? 3328 : 2816);
 }
 
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,

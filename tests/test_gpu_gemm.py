@@ -474,8 +474,8 @@ def test_small_grid_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     (515, 2050, 1024, False), (1025, 1000, 1408, False), (515, 2050, 1664, False), (1000, 1111, 1792, False),
     # 64 x 96 tiles, up to 128 tiles of 128 x 128 and beyond (K of whole stages, 2816 and more, 3328 and more)
     (1030, 1930, 1024, False), (1100, 1000, 1920, False), (2049, 1100, 1536, False), (1000, 3000, 2816, False), (1000, 3000, 3328, False),
-    # ... beyond, because 128 x 128 tiles would pad a quarter more
-    (130, 8500, 128, False), (130, 8500, 640, False),
+    # ... beyond, 64 x 64 tiles at every K
+    (130, 8500, 128, False), (577, 3270, 640, False), (1030, 1794, 1152, False),
     # shorter K on the form whose waves split every stage in two, with 64 x 64 and with 128 x 128 tiles
     (515, 2050, 128, False), (1025, 1000, 640, False), (1000, 1111, 1152, False), (1025, 1000, 1280, False),
     (1030, 1930, 128, False), (2049, 1100, 1152, False), (1000, 3000, 896, False), (1000, 3000, 3200, False),
