@@ -1163,18 +1163,22 @@ struct KSplit {
     unsigned *arrivals = nullptr;
 };
 
-// Whether the epilogue's operands get LDS: not where the CU would then hold fewer workgroups than it
-// has to run (a set-up call counts as none).  bf16 with bias, us, without that LDS / with: 32 x 28672 x 1536, two
-// workgroups of 80 KiB a CU or one, 8.0 / 9.75; 17 x 16640 x 1536 6.9 / 8.9; 40 x 65536 x 512, four or three,
-// 16.3 / 20.1.
+// Whether the epilogue's operands get LDS: not where all workgroups are on the device at once without it
+// and not with it (a set-up call counts as none).  bf16 with bias, us, without that LDS / with: 32 x 28672 x 1536,
+// 1.75 workgroups for each CU, which holds two or one of them, 8.0 / 9.75; 45 x 57344 x 512, four for four or three places, 14.3 /
+// 21.2; 17 x 122880 x 256, 7.5 for eight or seven, 9.4 / 12.4; but 45 x 90000 x 512, 5.5 for four or three, 25.7 / 22.1, 45 x
+// 63834 x 256, 15.6 for fourteen or twelve, 13.9 / 11.8, 29 x 73728 x 512, 4.5 for four either way, 10.7 / 9.5.
 bool early_epilogue(const Plan &p, int n, int slices)
 {
-    constexpr int kMaxWaves = 32;  // of a CU
+    constexpr int kMaxWaves = 32, kLdsGranule = 1280;  // of a CU: 160 KiB of LDS are handed out in 128 parts
     if (p.s == 0 || p.lds + kEpilogueBytes > kMaxLds)
         return false;
     const long workgroups = (long)((n + p.rows_blk - 1) / p.rows_blk) * slices;
-    const long wanted = std::min((long)(kMaxWaves / p.s), (workgroups + p.cus - 1) / p.cus);
-    return kMaxLds / (p.lds + kEpilogueBytes) >= std::min(wanted, (long)(kMaxLds / p.lds));
+    const auto at_once = [&](int lds) {
+        const int parts = (lds + kLdsGranule - 1) / kLdsGranule;
+        return workgroups <= (long)p.cus * std::min(kMaxLds / kLdsGranule / parts, kMaxWaves / p.s);
+    };
+    return at_once(p.lds + kEpilogueBytes) || !at_once(p.lds);
 }
 
 template <int T, int R, int FMX, bool XDMA, bool EPILOGUE>
