@@ -92,7 +92,7 @@ hipError_t set_up_device(PerDevice &pd, int dev)
 }
 
 // Set-up for the device that is current on the calling thread; returns its record.  Set-up
-// queries the device, raises the dynamic-LDS limit of some 250 kernels and takes the address
+// queries the device, raises the dynamic-LDS limit of some 400 kernels and takes the address
 // of the scratch arrays (which loads the device image): none of that belongs inside a graph
 // capture, so a first call that arrives with `work_stream` capturing is refused
 // (`for_work`: the call is about to enqueue work on work_stream).
@@ -129,13 +129,12 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 // The FP6 path pays off once its 256 x 256 tiles can occupy a good part of the device and K
 // is long enough to amortise the converter pass (a fixed cost of about (M + N) * K * 1.25
-// bytes of HBM traffic).  Measured against the int8 kernel (tiles, K -> faster kernel):
-// 128, 4096 -> tie; 128, 8192 -> FP6 by 8 %; 128, 14336 -> FP6 by 20 %; 144, 3072 -> FP6;
-// 256, 2048 -> int8 by 5 %; 512, 2048 -> FP6 by 20 %; 512, 1024 -> FP6 by 3 %; 1024, 1024
-// -> tie; 1024, 512 -> int8 by 10 %.  With 64 tiles or fewer the FP6 GEMM splits K, but the
-// int8 kernel's small-grid form is as fast or faster there (64 tiles: 62 against 81 us at
-// K = 14336, 122 against 131 and 115 against 109 us at K = 28672), so the automatic choice
-// leaves those shapes to it.
+// bytes of HBM traffic).  Measured against the int8 kernel (tiles, K: int8 / FP6 in us, back to back):
+// 128, 4096: 33.1 / 35.7; 128, 8192: 59.2 / 56.2; 128, 14336: 98.6 / 88.2; 144, 2048: 28.1 / 28.1;
+// 144, 3072: 40.5 / 32.6; 256, 2048: 37.1 / 37.0; 256, 3072: 49.4 / 42.9; 384, 1024: 39.5 / 38.6;
+// 512, 1024: 41.5 / 43.0; 512, 2048: 65.4 / 52.8; 1024, 1024: 77.1 / 64.3; 1024, 512: 56.2 / 58.2.  With 64
+// tiles or fewer the int8 kernel is the faster one at every K (64 tiles: 8192 32 / 48, 14336 52 / 70, 28672
+// 98 / 108).
 bool fp6_worthwhile(int m, int n, int k, const DeviceInfo &dev, size_t limit)
 {
     const long tiles = (long)((m + 255) / 256) * ((n + 255) / 256);

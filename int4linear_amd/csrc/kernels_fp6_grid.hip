@@ -7,9 +7,8 @@
 // which a CU pulls operands through its L1 (about 100 bytes per ns): 64 x 64 tiles read every operand
 // four times as often as 256 x 256 ones, which pays while those leave most of the device idle.
 // Measured against the large kernel (us, converter included): 333 x 1111 x 4104, 10 tiles of 256 x 256,
-// 33.2 -> 12.6; 256 x 1024 x 4096, 4 tiles, 28.3 -> 8.7 (graph); 512 x 4096 x 4096, 32 tiles, 25.0 ->
-// 15.9; 2048 x 2048 x 2048, 64 tiles, 21.4 -> 16.9; 1024 x 4096 x 4096, 64 tiles, 25.8 -> 24.4; 300 x
-// 14336 x 4096, 112 tiles, 28.7 -> 27.6.
+// 32.9 -> 12.6; 256 x 1024 x 4104, 4 tiles, 28.7 -> 10.3; 512 x 4096 x 4104, 32 tiles, 33.5 -> 25.1; 2048 x 2048 x
+// 2056, 64 tiles, 24.2 -> 23.3; 1024 x 4096 x 4104, 64 tiles, 32.3 -> 32.0; longer K: plan_gemm in kernels_fp6.hip.
 #include "fp6_format.h"
 #include "grid_tail.h"
 
@@ -182,7 +181,8 @@ hipError_t fp6_grid_init(const DeviceInfo &)
     return e;
 }
 
-// Up to four 64 x 64 tiles per CU, i.e. 256 x 256 tiles on a quarter of the CUs when they are whole.
+// Up to four 64 x 64 tiles per CU, i.e. 256 x 256 tiles on a quarter of the CUs when they are whole; long
+// K decides between the two in plan_gemm (kernels_fp6.hip).
 bool fp6_grid_preferred(int m, int n, const DeviceInfo &dev) { return grid_tiles(m, n, 64, 64) <= 4l * dev.cu_count; }
 
 // Slices of K across workgroups: the most that leave at most two workgroups per CU (they fit), 4096 k

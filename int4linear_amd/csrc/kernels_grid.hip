@@ -18,9 +18,10 @@
 //   * the epilogue's operands are fetched behind the first stage's loads, not after the last MFMA.
 //   * neighbouring columns of tiles start at different stages of K (the order of K does not
 //     matter to the sums), so that the CUs do not all miss on the same lines at the same time.
-// Measured against the 64 x 64 tile of four quadrants by two halves of K that it replaces, launches
-// from a graph: 65 x 4096 x 4096 9.5 -> 6.5 us, 333 x 1111 x 4096 9.6 -> 6.6, 256 x 4096 x 4096
-// 10.0 -> 9.1, 128 x 14336 x 4096 14.9 -> 13.0, 300 x 520 x 640 4.15 -> 3.7.
+// Measured against the 64 x 64 tile of four quadrants by two halves of K (mfma_pair64_kernel), back to back
+// on operands that stay in the caches: 65 x 4096 x 4096 9.3 -> 6.6 us, 333 x 1111 x 4096 9.3 -> 6.7, 256 x
+// 4096 x 4096 9.7 -> 8.5, 128 x 14336 x 4096 13.9 -> 12.2, 300 x 520 x 640 4.1 -> 3.7.  (Figures beside one
+// another are from one run; another machine, or a profiler, moves them by up to a third together.)
 //
 // With few tiles and long K a tile's K is split over workgroups as well; they exchange partial sums
 // through memory inside the same launch (see the kernel's end).
