@@ -1498,7 +1498,10 @@ bool make_ksplit_plan(int m, int n, int k, int cu_count, Plan &p, int &slices)
 // 16384 (the same with rotating outputs in parentheses): 64 x 2048 x 28672 13.4 / 12.8 (13.5 / 13.4), 64 x 3072 x 14336
 // 12.6 / 11.7 (12.6 / 11.9), 64 x 3072 x 16384 13.0 / 12.6 (13.0 / 12.9), 64 x 3072 x 24576 17.2 / 16.4 (17.2 / 16.8), 64 x
 // 4096 x 14336 13.2 / 12.4 (13.2 / 13.2; from the caches 12.4 / 10.9), but 64 x 4096 x 16384 13.9 / 13.2 (13.9 / 14.4), 64 x
-// 4096 x 28672 19.8 / 19.7 (20.0 / 21.4), 40 x 4096 x 14336 11.3 / 12.1, 40 x 2048 x 14336 8.6 / 9.3.
+// 4096 x 28672 19.8 / 19.7 (20.0 / 21.4), 40 x 4096 x 14336 11.3 / 12.1, 40 x 2048 x 14336 8.6 / 9.3.  As one of the seven
+// layers of a decode loop whose blocks have weights of their own, per block, 64 rows, bf16: 4096 x 14336 56.5 / 55.0, 3072 x
+// 14336 49.0 / 46.6, 3072 x 20480 69.7 / 67.1, 2048 x 28672 49.8 / 49.2.  (A launch by itself on a device that idles, all
+// of its memory cold, is the one that loses: 64 x 4096 x 14336 17.2 / 19.0.)
 bool tiles_split(int m, int n, int k, bool own_split, int slices)
 {  // (m <= 64)
     if (m <= 16 || slices <= 1)
