@@ -329,7 +329,7 @@ Tile choose_tile(int m, int n, int k, const DeviceInfo &dev)
 {
     if (grid_tiles(m, n, 32, 32) <= dev.cu_count)
         return Tile::k32x32;
-    if (grid_tiles(m, n, 64, 32) <= dev.cu_count)
+    if (grid_fits_narrow_tiles(m, n, dev))
         return k > 2048 ? Tile::k64x32Long : Tile::k64x32Short;
     const auto columns = [&](int bn) { return (grid_tiles(m, n, 64, bn) + dev.cu_count - 1) / dev.cu_count * bn; };
     return columns(64) < columns(96) ? Tile::k64x64 : Tile::k64x96;
@@ -455,6 +455,8 @@ bool grid_preferred(int m, int n, int k, const DeviceInfo &dev)
         return false;
     return m <= 64 || grid_tiles(m, n, 64, 64) <= 2l * dev.cu_count || long_enough(k, k % 512 == 128 ? 3328 : 2816);
 }
+
+bool grid_fits_narrow_tiles(int m, int n, const DeviceInfo &dev) { return grid_tiles(m, n, 64, 32) <= dev.cu_count; }
 
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
                        hipStream_t stream)

@@ -1168,8 +1168,11 @@ hipError_t launch_mfma_tile(const void *a, const void *b, void *c, int m, int n,
 // CUs at K >= 12288 (512 x 4096 x 14336 35.6 us split, 52 us as one tile per workgroup): the
 // largest divisor of the stage count that keeps at least eight stages per slice, at most eight
 // slices, and at most half a work item per slot.  Up to a quarter as many tiles as CUs the unsplit
-// small-grid form is as fast as two or three slices (512 x 2048 x 12672 21.4, 22.4 us in three), not as
-// more (300 x 2000 x 16000 25.0, 21.0 in five).
+// small-grid form is as fast as two or three slices (512 x 2048 x 12672 21.4, 22.4 us in three), and as
+// more while its 64 x 32 tiles number no more than the CUs (unsplit / five or seven slices, us: 707 x 261 x
+// 17024 13.9 / 17.4, 160 x 1216 x 17280 14.0 / 19.4, 254 x 1859 x 15232 16.1 / 18.9, 213 x 2004 x 23680, 252 of
+// them, 22.1 / 23.9).  Beyond, its tiles are 64 x 64 and the slices win: 327 x 1356 x 20608, 258 of them, 31.3 / 21.9,
+// 300 x 2000 x 16000 25.0 / 21.0, 922 x 666 x 16000 25.8 / 23.2.
 int mfma_ksplit(int m, int n, int k, const DeviceInfo &dev)
 {
     if (!mfma_supports(m, n, k))
@@ -1177,7 +1180,7 @@ int mfma_ksplit(int m, int n, int k, const DeviceInfo &dev)
     const long tiles = (long)((m + CfgMedium::BM - 1) / CfgMedium::BM) * ((n + CfgMedium::BN - 1) / CfgMedium::BN);
     const long slots = (long)dev.cu_count * CfgMedium::OCC;
     const int stages = k / kStageK;
-    if (tiles * 2 > dev.cu_count || tiles * 16 <= dev.cu_count || stages < 96)
+    if (tiles * 2 > dev.cu_count || grid_fits_narrow_tiles(m, n, dev) || stages < 96)
         return 1;
     long limit = slots / (2 * tiles);
     if (limit > 8)

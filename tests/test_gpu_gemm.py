@@ -479,6 +479,8 @@ def test_small_grid_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     # shorter K on the form whose waves split every stage in two, with 64 x 64 and with 128 x 128 tiles
     (515, 2050, 128, False), (1025, 1000, 640, False), (1000, 1111, 1152, False), (1025, 1000, 1280, False),
     (1030, 1930, 128, False), (2049, 1100, 1152, False), (1000, 3000, 896, False), (1000, 3000, 3200, False),
+    # long K that the slices do not divide: 64 x 32 tiles unsplit, up to one per CU
+    (160, 1216, 17280, False), (254, 1859, 15232, False),
     # each of them split over K across workgroups, with odd numbers of pieces per slice
     (65, 200, 8448, True), (200, 700, 8960, True), (250, 2300, 12544, True), (66, 60, 8320, True)])
 def test_tiles_of_the_small_grid_form(gpu, host_threads, m, n, k, split):
