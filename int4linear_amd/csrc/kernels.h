@@ -158,7 +158,7 @@ hipError_t launch_mfma_splitk(const void *a, const void *b, void *c, int m, int 
 // grid_split_bytes() bytes of partial sums in `workspace` (8-byte aligned; 0 = the shape is not
 // split), arrivals counted at `arrivals` as by launch_skinny_ksplit below.
 hipError_t grid_init(const DeviceInfo &dev);
-bool grid_preferred(int m, int n, int k, const DeviceInfo &dev);
+bool grid_preferred(int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev);
 bool grid_fits_narrow_tiles(int m, int n, const DeviceInfo &dev);  // at most one 64 x 32 tile per CU
 hipError_t launch_grid(const void *a, const void *b, void *c, int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev,
                        hipStream_t stream);

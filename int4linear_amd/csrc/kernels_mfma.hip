@@ -1240,7 +1240,7 @@ hipError_t launch_mfma(const void *a, const void *b, void *c, int m, int n, int 
     // Few 128 x 128 tiles per CU: the form whose two waves per SIMD split K.
     const int pair_m = (m + kPairTile - 1) / kPairTile, pair_n = (n + kPairTile - 1) / kPairTile;
     // ... and so few that smaller tiles leave the busiest CU less to do (kernels_grid.hip).
-    if (grid_preferred(m, n, k, dev))
+    if (grid_preferred(m, n, k, ep, dev))
         return launch_grid(a, b, c, m, n, k, ep, dev, stream);
     // ... with K too short for that form: 64 x 64 tiles where 128 x 128 ones would leave half of the CUs
     // idle or more (1024 x 1024 x 640 6.9 -> 4.6 us).

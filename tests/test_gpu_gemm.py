@@ -476,6 +476,8 @@ def test_small_grid_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     (1030, 1930, 1024, False), (1100, 1000, 1920, False), (2049, 1100, 1536, False), (1000, 3000, 2816, False), (1000, 3000, 3328, False),
     # ... beyond, 64 x 64 tiles at every K
     (130, 8500, 128, False), (577, 3270, 640, False), (1030, 1794, 1152, False),
+    # ... with a bias or scales in 32 bits from shorter K on
+    (1030, 1930, 384, False), (1000, 3000, 1152, False),
     # shorter K on the form whose waves split every stage in two, with 64 x 64 and with 128 x 128 tiles
     (515, 2050, 128, False), (1025, 1000, 640, False), (1000, 1111, 1152, False), (1025, 1000, 1280, False),
     (1030, 1930, 128, False), (2049, 1100, 1152, False), (1000, 3000, 896, False), (1000, 3000, 3200, False),
