@@ -351,7 +351,11 @@ bool long_enough(int k, int from)
 // CUs without work (32 x 32 and 64 x 32 tiles) or, with 64 x 64 tiles, a second workgroup fits every
 // CU.  The exchange costs some 2 us.  Measured, unsplit -> split: 200 x 136 x 16384 12.6 -> 7.9 us,
 // 300 x 520 x 12288 10.6 -> 10.0, 100 x 2000 x 16384 12.7 -> 11.6, 128 x 4096 x 28672 25.2 -> 22.3,
-// 128 x 4096 x 14336 14.8 -> 15.2 (nothing gained, nothing lost).
+// 128 x 4096 x 14336 14.8 -> 15.2 (nothing gained, nothing lost).  K that the few slices of the smaller
+// tiles do not divide goes to four and more slices of a larger one if it is long and they fit the CUs: 112 pieces
+// and more (us, unsplit / in five or seven slices: 242 x 133 x 17024 13.3 / 8.9, 229 x 329 x 15232 12.4 / 10.5, 299 x 553 x
+// 16000 12.85 / 11.85; more workgroups than CUs 104 x 1907 x 14720 12.6 / 13.1, three slices 119 x 1387 x 14976 12.5 /
+// 12.6 and with weights from HBM 12.5 / 16.1, shorter K 557 x 289 x 8832 8.65 / 10.2).
 struct SplitPlan {
     Tile tile = Tile::k64x64;
     int slices = 1;
@@ -360,28 +364,35 @@ struct SplitPlan {
 
 SplitPlan plan_split(int m, int n, int k, const DeviceInfo &dev)
 {
-    constexpr int kMinPieces = 64, kMinPiecesPerSlice = 8;
+    constexpr int kMinPieces = 64, kLongPieces = 112, kMinPiecesPerSlice = 8;
     SplitPlan p;
     const int pieces = k / kPieceK;
     if (pieces < kMinPieces)
         return p;
-    long tiles, most, waves, area;
-    if (grid_tiles(m, n, 32, 32) * 4 <= dev.cu_count) {
-        p.tile = Tile::k32x32;
-        tiles = grid_tiles(m, n, 32, 32), most = dev.cu_count, waves = Tile32x32::KG, area = 32 * 32;
-    } else if (grid_tiles(m, n, 64, 32) * 2 <= dev.cu_count) {
-        p.tile = Tile::k64x32Long;
-        tiles = grid_tiles(m, n, 64, 32), most = dev.cu_count, waves = Tile64x32Long::KG, area = 64 * 32;
-    } else {
-        tiles = grid_tiles(m, n, 64, 64), most = 2l * dev.cu_count, waves = Tile64x64::KG, area = 64 * 64;
-    }
-    if (tiles * waves > kSkinnyArrivalWords)
-        return p;
-    for (int d = 2; d <= kGridMaxSlices && tiles * d <= most; ++d)
-        if (pieces % d == 0 && pieces / d >= kMinPiecesPerSlice)
-            p.slices = d;
-    if (p.slices > 1)
-        p.bytes = (size_t)tiles * p.slices * area * 4;
+    // (`least`, `most`: slices and workgroups)
+    const auto split = [&](Tile tile, int bm, int bn, int waves, int least, long most) {
+        const long tiles = grid_tiles(m, n, bm, bn);
+        if (tiles * waves > kSkinnyArrivalWords)
+            return;
+        for (int d = least; d <= kGridMaxSlices && tiles * d <= most; ++d)
+            if (pieces % d == 0 && pieces / d >= kMinPiecesPerSlice) {
+                p.tile = tile;
+                p.slices = d;
+                p.bytes = (size_t)tiles * d * bm * bn * 4;
+            }
+    };
+    const int cus = dev.cu_count;
+    const bool tiles32 = grid_tiles(m, n, 32, 32) * 4 <= cus, tiles64x32 = grid_tiles(m, n, 64, 32) * 2 <= cus;
+    if (tiles32)
+        split(Tile::k32x32, 32, 32, Tile32x32::KG, 2, cus);
+    else if (tiles64x32)
+        split(Tile::k64x32Long, 64, 32, Tile64x32Long::KG, 2, cus);
+    else
+        split(Tile::k64x64, 64, 64, Tile64x64::KG, 2, 2l * cus);
+    if (p.slices == 1 && pieces >= kLongPieces && tiles32)
+        split(Tile::k64x32Long, 64, 32, Tile64x32Long::KG, 4, cus);
+    if (p.slices == 1 && pieces >= kLongPieces && tiles64x32)
+        split(Tile::k64x64, 64, 64, Tile64x64::KG, 4, cus);
     return p;
 }
 

@@ -484,7 +484,9 @@ def test_small_grid_form_of_the_int8_kernel(gpu, host_threads, m, n, k):
     # long K that the slices do not divide: 64 x 32 tiles unsplit, up to one per CU
     (160, 1216, 17280, False), (254, 1859, 15232, False),
     # each of them split over K across workgroups, with odd numbers of pieces per slice
-    (65, 200, 8448, True), (200, 700, 8960, True), (250, 2300, 12544, True), (66, 60, 8320, True)])
+    (65, 200, 8448, True), (200, 700, 8960, True), (250, 2300, 12544, True), (66, 60, 8320, True),
+    # ... long K that only slices of the next larger tile divide: 64 x 32 and 64 x 64; too many of them for the CUs
+    (242, 133, 15232, True), (211, 317, 16000, True), (470, 264, 15232, False)])
 def test_tiles_of_the_small_grid_form(gpu, host_threads, m, n, k, split):
     """Every tile of the small-grid form at its edges, and the forms that take shorter K: rows and
     columns past the tile, K that ends inside a stage, fewer stages than the ring holds, all output
