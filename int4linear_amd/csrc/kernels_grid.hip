@@ -456,10 +456,11 @@ hipError_t grid_init(const DeviceInfo &)
 // 64 rows, half of what its tiles hold, and where 64 x 64 tiles fit the device two to a CU (int32, us, that
 // kernel / this one: 700 x 2712, 473 of them, x 256 6.8 / 6.0, x 1152 8.9 / 7.7; 257 x 5464, 430, x 1920 10.5 / 8.2), so
 // that they are the ones chosen; with 64 x 96 tiles once K is long enough (580 x 3500 x 640 7.5 / 8.5), which is
-// sooner where C is written in 32 bits and has a bias or scales, at the cost of which that kernel's tiles end later
+// sooner where C is written in 32 bits and has a bias or scales, which end that kernel's tiles later
 // (with a bias: 386 x 6470 x 512 9.4 / 8.4, 418 x 4705 x 896 9.3 / 8.4, 1161 x 2474 x 640 9.7 / 9.3, 2009 x 1444 x 384 9.0 /
 // 8.5, x 1152 equal, 429 x 5383 x 1792 12.7 / 11.6; float output: 924 x 2594 x 640 9.35 / 9.8, 424 x 5377 x 1152 equal, 410 x
-// 5392 x 1280 11.05 / 10.6, 807 x 2734 x 2432 15.0 / 13.5; without, and in 16 bits, to the line above: 309 x 9099 x 1280 10.1 / 10.4).
+// 5392 x 1280 11.05 / 10.6, 807 x 2734 x 2432 15.0 / 13.5, whole stages 619 x 4252 x 512 9.3 / 8.85; without either, and in 16 bits,
+// that line stays: 309 x 9099 x 1280 10.1 / 10.4).
 bool grid_preferred(int m, int n, int k, const Epilogue &ep, const DeviceInfo &dev)
 {
     if (few_tiles(m, n, dev)) {
@@ -471,7 +472,7 @@ bool grid_preferred(int m, int n, int k, const Epilogue &ep, const DeviceInfo &d
     if (m <= 64 || grid_tiles(m, n, 64, 64) <= 2l * dev.cu_count)
         return true;
     if (ep.out == kOutF32)
-        return long_enough(k, 1152);
+        return k >= 1152 || k % 512 == 0;
     if (ep.out == kOutS32 && ep.bias)
         return k >= 384;
     return long_enough(k, k % 512 == 128 ? 3328 : 2816);
