@@ -17,7 +17,8 @@
 //     are shifted and masked.  No registers for a second set, so three waves fit a SIMD.
 //   * the epilogue's operands are fetched behind the first stage's loads, not after the last MFMA.
 //   * neighbouring columns of tiles start at different stages of K (the order of K does not
-//     matter to the sums), so that the CUs do not all miss on the same lines at the same time.
+//     matter to the sums), so that the CUs do not all miss on the same lines at the same time.  (All at
+//     the first: 120 shapes on the larger tiles within 5 % either way, 0.2 % on average.)
 // Measured against the 64 x 64 tile of four quadrants by two halves of K (mfma_pair64_kernel), back to back
 // on operands that stay in the caches: 65 x 4096 x 4096 9.3 -> 6.6 us, 333 x 1111 x 4096 9.3 -> 6.7, 256 x
 // 4096 x 4096 9.7 -> 8.5, 128 x 14336 x 4096 13.9 -> 12.2, 300 x 520 x 640 4.1 -> 3.7.  (Figures beside one
