@@ -677,6 +677,9 @@ int large_slices(long tiles, int stages, const DeviceInfo &dev)
 // 28672 161 / 116 (4) / -; 768 x 3072 x 16376 72 / 55 (4) / -; 1000 x 3000 x 12296 58 / - / 67; 512 x 4096 x 16384
 // 60 / 73 (8) / -, x 28680 98 / 80 (5) / -; 600 x 3300 x 28680 121 / 89 (5) / -.  Unsplit 256 x 256 tiles fall behind
 // again once the operands outgrow the memory-side cache (512 x 8192 x 24584, 160 MB: 158 / - / 161; x 32776 252 / - / 281).
+// Rows of C that are no multiple of 4 long are stored and added up a dword at a time: 64 x 64 / slices, 2026 x 1819 x 10728
+// 68 / 87 (4), 256 x 13066 x 10232 80 / 95 (4), 2692 x 1086 x 14240 68 / 82 (4), though 482 x 6845 x 14888 96 / 84 (3); a
+// multiple of 4: 4743 x 704 x 13016 82 / 69 (3), 1482 x 2220 x 12256 75 / 70 (4).  (The converter is in these times.)
 GemmPlan plan_gemm(int m, int n, int k, const DeviceInfo &dev, size_t room)
 {
     constexpr size_t kCachedOperands = 140u << 20;
@@ -693,7 +696,8 @@ GemmPlan plan_gemm(int m, int n, int k, const DeviceInfo &dev, size_t room)
         const double whole = cached ? 10 + per_k : small;
         const int d = large_slices(tiles, stages, dev);
         const size_t slabs = (size_t)d * (size_t)m * (size_t)n * 4u;
-        const double split = d > 1 && slabs <= room ? 10 + per_k / d + (2 * d + 1) * 4. * m * n / 4.5e6 : small;
+        const double slab_rate = n % 4 == 0 ? 4.2e6 : 2.8e6;  // bytes per us
+        const double split = d > 1 && slabs <= room ? 10 + per_k / d + (2 * d + 1) * 4. * m * n / slab_rate : small;
         if (split < small && split <= whole)
             return GemmPlan{false, d, slabs};
         if (whole < small)

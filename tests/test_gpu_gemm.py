@@ -795,7 +795,8 @@ def test_fp6_forms_and_their_workspace(gpu, host_threads):
         pytest.skip("the sizes below are those of 256 compute units")
     operands = lambda m, n, k: lib.fp6_operand_bytes(m, k) + lib.fp6_operand_bytes(n, k)
     for (m, n, k), slices in (((1024, 4096, 16376), 4), ((600, 3301, 16376), 4), ((512, 4096, 28680), 5), ((1536, 2560, 28680), 3),
-                              ((1024, 4096, 12296), 0), ((512, 4096, 16376), 0), ((1000, 3000, 4104), 0)):
+                              ((1024, 4096, 12296), 0), ((512, 4096, 16376), 0), ((1000, 3000, 4104), 0),
+                              ((2026, 1819, 10728), 0), ((256, 13066, 10232), 0), ((1482, 2220, 12256), 4)):
         assert lib.workspace_bytes(m, n, k) == operands(m, n, k) + slices * m * n * 4, (m, n, k)
     m, n, k = 600, 3301, 16376
     x, w = helpers.uniform_s4(3800, m, k), helpers.uniform_s4(3801, n, k)
